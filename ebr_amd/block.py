@@ -19,7 +19,7 @@ from typing import Tuple
 import torch
 from torch.autograd.function import once_differentiable
 
-from ebr_amd import _capi
+from ebr_amd import _capi, _host
 from ebr_amd.fused_attn.loader import hip_library
 from ebr_amd.fused_attn.ops import _DTYPE_CODE, _stream
 
@@ -266,11 +266,19 @@ class _SwiGLU(torch.autograd.Function):
 
 def rms_norm(x: Tensor, eps: float) -> Tensor:
     """Unit RMS over the last dim (statistics in fp32), differentiable twice."""
+    host = _host.module()
+    y = None if host is None else host.rms_norm(x, eps)
+    if y is not None:
+        return y
     return _RmsNorm.apply(x, eps)
 
 
 def swiglu(gate_up: Tensor) -> Tensor:
     """silu(gate) * up of the two halves of the last dim, differentiable twice."""
+    host = _host.module()
+    y = None if host is None else host.swiglu(gate_up)
+    if y is not None:
+        return y
     _half(gate_up)
     return _SwiGLU.apply(gate_up)
 

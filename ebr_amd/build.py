@@ -1,6 +1,7 @@
-"""Build recipe of the gfx950 HIP library ``ebr_amd/_lib/libebr_attn.so`` (in-tree, so it travels with the repo).
+"""Build recipe of the gfx950 HIP library ``ebr_amd/_lib/libebr_attn.so`` and of the native host path
+``ebr_amd/_lib/ebr_host.so`` (both in-tree, so they travel with the repo).
 
-``python -m ebr_amd.build`` compiles it; ``__graft_entry__.build()`` calls :func:`build`. hipcc cross-compiles for
+``python -m ebr_amd.build`` compiles them; ``__graft_entry__.build()`` calls :func:`build` and :func:`build_host`. hipcc cross-compiles for
 gfx950 without a GPU. Packed-fp32 instruction selection is disabled (``-packed-fp32-ops``) for every HIP source.
 """
 
@@ -10,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import time
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -19,6 +21,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 OUT_DIR = PKG / "_lib"
 LIB_NAME = "libebr_attn.so"
+HOST_NAME = "ebr_host.so"
 ARCH = "gfx950"
 
 SOURCES = [CSRC / "ebr_attn.hip", CSRC / "ebr_rope.hip", CSRC / "ebr_descent.hip", CSRC / "ebr_block.hip",
@@ -72,7 +75,7 @@ def _run(cmd: list, verbose: bool) -> str:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         sys.stderr.write(proc.stdout + proc.stderr)
-        raise RuntimeError(f"hipcc failed with exit code {proc.returncode}: {' '.join(cmd[-3:])}")
+        raise RuntimeError(f"{Path(cmd[0]).name} failed with exit code {proc.returncode}: {' '.join(cmd[-3:])}")
     return proc.stderr
 
 
@@ -104,5 +107,48 @@ def build(verbose: bool = False, extra_flags: tuple = (), jobs: int = 0, arch: s
     return out
 
 
+def host_command(out: Path) -> list:
+    """The host compiler's command for the native host path: torch's headers and libraries, the library's own ABI."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    incs = [ROOT / "include", *include_paths(), rocm / "include", sysconfig.get_paths()["include"]]
+    libs = ["torch_python", "torch", "torch_cpu", "c10", "c10_hip", "ebr_attn"]
+    return [
+        os.environ.get("CXX", "g++"),
+        "-O2",
+        "-std=c++17",
+        "-shared",
+        "-fPIC",
+        "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1",
+        "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *(f"-I{i}" for i in incs),
+        str(CSRC / "ebr_host.cpp"),
+        f"-L{lib}",
+        f"-L{OUT_DIR}",
+        *(f"-l{n}" for n in libs),
+        "-Wl,-rpath,$ORIGIN",
+        "-o",
+        str(out),
+    ]
+
+
+def build_host(verbose: bool = False) -> Path:
+    """Compile the native host path against the built library and this interpreter's torch; return its path."""
+    out = OUT_DIR / HOST_NAME
+    tmp = out.with_suffix(".so.tmp")
+    t0 = time.time()
+    _run(host_command(tmp), verbose)
+    os.replace(tmp, out)
+    if verbose:
+        print(f"host path built in {time.time() - t0:.1f} s", flush=True)
+    return out
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_host(verbose=True))

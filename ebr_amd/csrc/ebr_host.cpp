@@ -1,0 +1,778 @@
+// Native host path of the GPU ops: argument checks, output allocation, autograd nodes and the launches of
+// libebr_attn.so (include/ebr_*.h) in C++, for calls on plain GPU tensors.
+//
+// The Python layer (ebr_amd/fused_attn/ops.py, rope_split.py, block.py, descent.py, linear.py) defines the ops, their
+// fakes and their autograd Functions, and stays the path of every call this file does not take: tensor subclasses and
+// fake tensors, torch.func transforms, dispatch and function modes, tracing, forward-mode duals, saved-tensor hooks,
+// tensors off the GPU, and every argument the Python layer would refuse or pad. Each entry point below returns None for
+// those, and the caller goes on in Python.
+//
+// Why it exists: a graded attention step (three launches) spent 453 us on the host in Python (autograd Functions,
+// custom-op dispatch, ctypes marshalling, GIL hand-overs to the engine's threads) against 45 us of kernel time for one
+// board and 310 us for the 768-board batch. The same nodes without Python take 140 us, of which two empty trips through
+// torch's autograd engine are 66.
+//
+// Nothing is kept between calls: outputs and scratch come from torch's allocator on the current stream, launches go to
+// the current stream of the tensors' device, and the nodes hold saved tensors through torch's SavedVariable only.
+#include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
+#include <ATen/record_function.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+
+#include "ebr_attn.h"
+#include "ebr_block.h"
+#include "ebr_descent.h"
+#include "ebr_rope.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+namespace py = pybind11;
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Which calls are taken
+// ---------------------------------------------------------------------------------------------------------------------
+
+// No mode, transform, tracer or saved-tensor hook that has to see the ops or their saved tensors.
+bool plain_context() {
+    return !at::impl::torch_function_mode_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize) &&
+           !torch::jit::tracer::isTracing() && !at::SavedTensorDefaultHooks::get_hooks().has_value();
+}
+
+// The tensor behind a Python argument if it is an ordinary dense GPU tensor, else an undefined one.
+Tensor plain(const py::handle& h) {
+    if (!THPVariable_CheckExact(h.ptr())) return {};
+    const Tensor& t = THPVariable_Unpack(h.ptr());
+    static const c10::DispatchKeySet allowed({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
+                                              c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
+    if (!t.defined() || !t.is_cuda() || (t.key_set().raw_repr() & ~allowed.raw_repr()) != 0 || t.is_inference())
+        return {};
+    if (t._fw_grad(/*level=*/0).defined()) return {};
+    return t;
+}
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return EBR_DTYPE_F32;
+        case at::kBFloat16: return EBR_DTYPE_BF16;
+        case at::kHalf: return EBR_DTYPE_F16;
+        case at::kDouble: return EBR_DTYPE_F64;
+        default: return -1;
+    }
+}
+
+bool same_kind(const Tensor& a, const Tensor& b) {
+    return a.scalar_type() == b.scalar_type() && a.device() == b.device();
+}
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+void check(int rc, const char* what) {
+    if (rc == 0) return;
+    TORCH_CHECK_TYPE(rc != EBR_ERR_DTYPE, what, ": ", ebr_attn_error_string(rc), " (code ", rc, ")");
+    TORCH_CHECK_VALUE(rc != EBR_ERR_SHAPE, what, ": ", ebr_attn_error_string(rc), " (code ", rc, ")");
+    TORCH_CHECK(false, what, ": ", ebr_attn_error_string(rc), " (code ", rc, ")");
+}
+
+// Outputs of a backward that is not differentiable again, for a derivative that is recorded: as torch's
+// once_differentiable, an error when a later backward reaches them.
+variable_list last(variable_list outs) {
+    variable_list in;
+    std::vector<size_t> at_;
+    for (size_t i = 0; i < outs.size(); ++i)
+        if (outs[i].defined()) {
+            in.push_back(outs[i].detach().set_requires_grad(true));
+            at_.push_back(i);
+        }
+    const auto err = std::make_shared<torch::autograd::DelayedError>(
+        "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)in.size());
+    const variable_list out = err->apply(std::move(in));
+    for (size_t i = 0; i < at_.size(); ++i) outs[at_[i]] = out[i];
+    return outs;
+}
+
+// An operand that a call may lack, as an autograd node takes it.
+std::optional<Tensor> maybe(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
+
+bool recorded(std::initializer_list<Tensor> ts) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor& t : ts)
+        if (t.defined() && t.requires_grad()) return true;
+    return false;
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Attention
+// ---------------------------------------------------------------------------------------------------------------------
+
+struct Str3 {
+    int64_t s[3];
+    explicit Str3(const Tensor& t) : s{t.stride(0), t.stride(1), t.stride(2)} {}
+};
+
+// Any B/H/L strides whose row starts are 16-byte aligned, with unit D stride; else a contiguous copy.
+Tensor rows(const Tensor& t) {
+    const int64_t es = t.element_size();
+    bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    for (int i = 0; i < 3; ++i) ok = ok && t.stride(i) >= 0 && (t.stride(i) * es) % 16 == 0;
+    return ok ? t : t.contiguous();
+}
+
+Tensor contig(const Tensor& t) {
+    return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0
+               ? t
+               : t.clone(at::MemoryFormat::Contiguous);
+}
+
+struct Dims {
+    int B, H, L, D;
+    explicit Dims(const Tensor& q)
+        : B((int)q.size(0)), H((int)q.size(1)), L((int)q.size(2)), D((int)q.size(3)) {}
+};
+
+Tensor scratch(int op, const Tensor& q) {
+    const Dims d(q);
+    const int64_t n = ebr_attn_scratch_bytes(op, d.B, d.H, d.L, d.D);
+    return n > 0 ? at::empty({(n + 3) / 4}, q.options().dtype(at::kFloat)) : Tensor();
+}
+
+float* fptr(const Tensor& t) { return t.defined() ? static_cast<float*>(t.data_ptr()) : nullptr; }
+
+variable_list attn_fwd(const Tensor& q_, const Tensor& k_, const Tensor& v_, double scale) {
+    RECORD_FUNCTION("ebr_fused::attn_fwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(q_.device());
+    const Tensor q = rows(q_), k = rows(k_), v = rows(v_);
+    const Dims d(q);
+    const Tensor o = at::empty(q.sizes(), q.options());
+    const Tensor lse = at::empty({d.B, d.H, d.L}, q.options().dtype(at::kFloat));
+    check(ebr_attn_fwd(dtype_code(q.scalar_type()), d.B, d.H, d.L, d.D, (float)scale, q.data_ptr(), Str3(q).s,
+                       k.data_ptr(), Str3(k).s, v.data_ptr(), Str3(v).s, o.data_ptr(), lse.data_ptr(), stream_of(q)),
+          "ebr_attn_fwd");
+    return {o, lse};
+}
+
+variable_list attn_bwd(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_, const Tensor& lse_,
+                       const Tensor& do_, double scale) {
+    RECORD_FUNCTION("ebr_fused::attn_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(q_.device());
+    const Tensor q = rows(q_), k = rows(k_), v = rows(v_), dO = rows(do_.to(q_.scalar_type()));
+    const Tensor o = contig(o_), lse = contig(lse_);
+    const Dims d(q);
+    variable_list out(3);
+    for (Tensor& t : out) t = at::empty(q.sizes(), q.options());
+    const Tensor s = scratch(EBR_OP_BWD, q);
+    check(ebr_attn_bwd(dtype_code(q.scalar_type()), d.B, d.H, d.L, d.D, (float)scale, q.data_ptr(), Str3(q).s,
+                       k.data_ptr(), Str3(k).s, v.data_ptr(), Str3(v).s, o.data_ptr(), lse.data_ptr(), dO.data_ptr(),
+                       Str3(dO).s, out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), fptr(s), stream_of(q)),
+          "ebr_attn_bwd");
+    return out;
+}
+
+variable_list attn_bwd_bwd(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_,
+                           const Tensor& lse_, const Tensor& do_, const Tensor& gq_, const Tensor& gk_,
+                           const Tensor& gv_, double scale) {
+    RECORD_FUNCTION("ebr_fused::attn_bwd_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(q_.device());
+    const auto st = q_.scalar_type();
+    const Tensor q = rows(q_), k = rows(k_), v = rows(v_), dO = rows(do_.to(st));
+    const Tensor gq = rows(gq_.to(st)), gk = rows(gk_.to(st)), gv = rows(gv_.to(st));
+    const Tensor o = contig(o_), lse = contig(lse_);
+    const Dims d(q);
+    variable_list out(4);
+    for (Tensor& t : out) t = at::empty(q.sizes(), q.options());
+    const Tensor s = scratch(EBR_OP_BWD_BWD, q);
+    check(ebr_attn_bwd_bwd(dtype_code(st), d.B, d.H, d.L, d.D, (float)scale, q.data_ptr(), Str3(q).s, k.data_ptr(),
+                           Str3(k).s, v.data_ptr(), Str3(v).s, o.data_ptr(), lse.data_ptr(), dO.data_ptr(),
+                           Str3(dO).s, gq.data_ptr(), Str3(gq).s, gk.data_ptr(), Str3(gk).s, gv.data_ptr(),
+                           Str3(gv).s, out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), out[3].data_ptr(),
+                           fptr(s), stream_of(q)),
+          "ebr_attn_bwd_bwd");
+    return out;
+}
+
+struct AttnBwdBwd : Function<AttnBwdBwd> {
+    static variable_list forward(AutogradContext*, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                 const Tensor& lse, const Tensor& dO, const Tensor& gq, const Tensor& gk,
+                                 const Tensor& gv, double scale) {
+        return attn_bwd_bwd(q, k, v, o, lse, dO, gq, gk, gv, scale);
+    }
+    static variable_list backward(AutogradContext*, const variable_list&) {
+        TORCH_CHECK(false, "ebr_fused::attn_bwd_bwd has no derivative");
+    }
+};
+
+// First derivative as a differentiable node; o and lse are constants in it (their dependence is in hq, hk, hv, hdo).
+struct AttnBwd : Function<AttnBwd> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                                 const Tensor& o, const Tensor& lse, const Tensor& dO, double scale) {
+        ctx->save_for_backward({q, k, v, o, lse, dO});
+        ctx->saved_data["scale"] = scale;
+        ctx->set_materialize_grads(false);  // an unused output's cotangent becomes one expanded zero row
+        return attn_bwd(q, k, v, o, lse, dO, scale);
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        const variable_list s = ctx->get_saved_variables();
+        const double scale = ctx->saved_data["scale"].toDouble();
+        Tensor cot[3];
+        for (int i = 0; i < 3; ++i)
+            cot[i] = g[i].defined() ? g[i] : at::zeros({s[i].size(3)}, s[i].options()).expand(s[i].sizes());
+        const variable_list h =
+            recorded({s[0], s[1], s[2], s[5], cot[0], cot[1], cot[2]})
+                ? AttnBwdBwd::apply(s[0], s[1], s[2], s[3], s[4], s[5], cot[0], cot[1], cot[2], scale)
+                : attn_bwd_bwd(s[0], s[1], s[2], s[3], s[4], s[5], cot[0], cot[1], cot[2], scale);
+        return {h[0], h[1], h[2], Tensor(), Tensor(), h[3].to(s[5].scalar_type()), Tensor()};
+    }
+};
+
+struct AttnFwd : Function<AttnFwd> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                                 double scale) {
+        variable_list out = attn_fwd(q, k, v, scale);
+        ctx->mark_non_differentiable({out[1]});
+        ctx->save_for_backward({q, k, v, out[0], out[1]});
+        ctx->saved_data["scale"] = scale;
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(4);  // only AttnBwd used o: nothing to add
+        const variable_list s = ctx->get_saved_variables();
+        variable_list d = AttnBwd::apply(s[0], s[1], s[2], s[3], s[4], g[0], ctx->saved_data["scale"].toDouble());
+        d.emplace_back();
+        return d;
+    }
+};
+
+// fused_attention, or None for a call that stays in Python.
+py::object attention(const py::handle& hq, const py::handle& hk, const py::handle& hv, std::optional<double> scale) {
+    const Tensor q = plain(hq), k = plain(hk), v = plain(hv);
+    if (!q.defined() || !k.defined() || !v.defined() || !plain_context()) return py::none();
+    if (q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes() || !same_kind(q, k) || !same_kind(q, v))
+        return py::none();
+    const int code = dtype_code(q.scalar_type());
+    if (code < 0 || code == EBR_DTYPE_F64 || q.numel() == 0) return py::none();
+    const int64_t D = q.size(3);
+    if (D > 256 || D % (code == EBR_DTYPE_F32 ? 4 : 8) || q.numel() / D >= (int64_t(1) << 31)) return py::none();
+    return py::cast(AttnFwd::apply(q, k, v, scale ? *scale : 1.0 / std::sqrt((double)D))[0]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// RoPE split and merge: each other's adjoint; the tables and the temperature carry no gradient
+// ---------------------------------------------------------------------------------------------------------------------
+
+Tensor unit_last(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+
+variable_list rope_split_launch(const Tensor& qkv_, const Tensor& cos, const Tensor& sin, const Tensor& qs,
+                                int64_t heads) {
+    RECORD_FUNCTION("ebr_fused::rope_split", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(qkv_.device());
+    const Tensor qkv = unit_last(qkv_);
+    const int64_t B = qkv.size(0), N = qkv.size(1), D = qkv.size(2) / (3 * heads);
+    variable_list out(3);
+    for (Tensor& t : out) t = at::empty({B, heads, N, D}, qkv.options());
+    check(ebr_rope_split(dtype_code(qkv.scalar_type()), (int)B, (int)N, (int)heads, (int)D, qkv.data_ptr(),
+                         qkv.stride(0), qkv.stride(1), fptr(cos), fptr(sin), fptr(qs), out[0].data_ptr(),
+                         out[1].data_ptr(), out[2].data_ptr(), stream_of(qkv)),
+          "ebr_rope_split");
+    return out;
+}
+
+Tensor rope_merge_launch(const Tensor& dq_, const Tensor& dk_, const Tensor& dv_, const Tensor& cos,
+                         const Tensor& sin, const Tensor& qs) {
+    RECORD_FUNCTION("ebr_fused::rope_merge", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(dq_.device());
+    const auto st = dq_.scalar_type();
+    const Tensor dq = unit_last(dq_), dk = unit_last(dk_.to(st)), dv = unit_last(dv_.to(st));
+    const Dims d(dq);
+    const Tensor g = at::empty({d.B, d.L, int64_t(3) * d.H * d.D}, dq.options());
+    check(ebr_rope_merge(dtype_code(st), d.B, d.H, d.L, d.D, dq.data_ptr(), Str3(dq).s, dk.data_ptr(), Str3(dk).s,
+                         dv.data_ptr(), Str3(dv).s, fptr(cos), fptr(sin), fptr(qs), g.data_ptr(), stream_of(dq)),
+          "ebr_rope_merge");
+    return g;
+}
+
+struct RopeMerge;
+
+struct RopeSplit : Function<RopeSplit> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin,
+                                 const std::optional<Tensor>& qs_, int64_t heads) {
+        const Tensor qs = qs_.value_or(Tensor());
+        ctx->save_for_backward({cos, sin, qs});
+        ctx->set_materialize_grads(false);
+        variable_list out = rope_split_launch(qkv, cos, sin, qs, heads);
+        ctx->saved_data["shape"] = out[0].sizes().vec();
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g);
+};
+
+struct RopeMerge : Function<RopeMerge> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& dq, const Tensor& dk, const Tensor& dv,
+                                 const Tensor& cos, const Tensor& sin, const std::optional<Tensor>& qs_) {
+        const Tensor qs = qs_.value_or(Tensor());
+        ctx->save_for_backward({cos, sin, qs});
+        ctx->saved_data["heads"] = dq.size(1);
+        ctx->set_materialize_grads(false);
+        return {rope_merge_launch(dq, dk, dv, cos, sin, qs)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(6);
+        const variable_list s = ctx->get_saved_variables();
+        variable_list d = RopeSplit::apply(g[0], s[0], s[1], maybe(s[2]), ctx->saved_data["heads"].toInt());
+        d.resize(6);
+        return d;
+    }
+};
+
+variable_list RopeSplit::backward(AutogradContext* ctx, const variable_list& g) {
+    variable_list out(5);
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    Tensor some;
+    for (const Tensor& t : g)
+        if (t.defined()) some = t;
+    if (!some.defined()) return out;
+    Tensor d[3];
+    for (int i = 0; i < 3; ++i) d[i] = g[i].defined() ? g[i] : at::zeros({shape[3]}, some.options()).expand(shape);
+    const variable_list s = ctx->get_saved_variables();
+    out[0] = RopeMerge::apply(d[0], d[1], d[2], s[0], s[1], maybe(s[2]))[0];
+    return out;
+}
+
+py::object rope_split(const py::handle& hqkv, const py::handle& hcos, const py::handle& hsin, int64_t heads,
+                      const py::handle& hqs) {
+    const Tensor qkv = plain(hqkv);
+    Tensor cos = plain(hcos), sin = plain(hsin), qs;
+    if (!qkv.defined() || !cos.defined() || !sin.defined() || !plain_context()) return py::none();
+    if (!hqs.is_none()) {
+        qs = plain(hqs);
+        if (!qs.defined() || qs.numel() != heads || qs.device() != qkv.device()) return py::none();
+        qs = qs.detach().to(at::kFloat).contiguous();
+    }
+    const int code = dtype_code(qkv.scalar_type());
+    if (code < 0 || code == EBR_DTYPE_F64 || heads < 1 || qkv.dim() != 3 || qkv.numel() == 0 ||
+        qkv.size(2) % (3 * heads))
+        return py::none();
+    const int64_t N = qkv.size(1), D = qkv.size(2) / (3 * heads);
+    const std::vector<int64_t> table = {N, D};
+    if (D % 4 || D > 256 || cos.sizes() != table || sin.sizes() != table || cos.device() != qkv.device() ||
+        sin.device() != qkv.device())
+        return py::none();
+    cos = cos.to(at::kFloat).contiguous();
+    sin = sin.to(at::kFloat).contiguous();
+    const variable_list o = RopeSplit::apply(qkv, cos, sin, maybe(qs), heads);
+    return py::make_tuple(o[0], o[1], o[2]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Energy block: rms_norm and SwiGLU, each differentiable twice
+// ---------------------------------------------------------------------------------------------------------------------
+
+Tensor dense(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+
+struct RowsOf {
+    int64_t rows, width;
+    explicit RowsOf(const Tensor& t) : rows(t.numel() / t.size(-1)), width(t.size(-1)) {}
+};
+
+Tensor rmsnorm(const Tensor& x_, double eps) {
+    RECORD_FUNCTION("ebr_fused::block_rmsnorm", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(x_.device());
+    const Tensor x = dense(x_), y = at::empty(x.sizes(), x.options());
+    const RowsOf r(x);
+    check(ebr_block_rmsnorm(dtype_code(x.scalar_type()), r.rows, (int)r.width, (float)eps, x.data_ptr(), y.data_ptr(),
+                            stream_of(x)),
+          "ebr_block_rmsnorm");
+    return y;
+}
+
+Tensor rmsnorm_bwd(const Tensor& x_, const Tensor& dy_, double eps) {
+    RECORD_FUNCTION("ebr_fused::block_rmsnorm_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(x_.device());
+    const Tensor x = dense(x_), dy = dense(dy_.to(x_.scalar_type())), dx = at::empty(x.sizes(), x.options());
+    const RowsOf r(x);
+    check(ebr_block_rmsnorm_bwd(dtype_code(x.scalar_type()), r.rows, (int)r.width, (float)eps, x.data_ptr(),
+                                dy.data_ptr(), dx.data_ptr(), stream_of(x)),
+          "ebr_block_rmsnorm_bwd");
+    return dx;
+}
+
+variable_list rmsnorm_bwd2(const Tensor& x_, const Tensor& dy_, const Tensor& c_, double eps) {
+    RECORD_FUNCTION("ebr_fused::block_rmsnorm_bwd2", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(x_.device());
+    const auto st = x_.scalar_type();
+    const Tensor x = dense(x_), dy = dense(dy_.to(st)), c = dense(c_.to(st));
+    const Tensor gx = at::empty(x.sizes(), x.options()), gdy = at::empty(x.sizes(), x.options());
+    const RowsOf r(x);
+    check(ebr_block_rmsnorm_bwd2(dtype_code(st), r.rows, (int)r.width, (float)eps, x.data_ptr(), dy.data_ptr(),
+                                 c.data_ptr(), gx.data_ptr(), gdy.data_ptr(), stream_of(x)),
+          "ebr_block_rmsnorm_bwd2");
+    return {gx, gdy};
+}
+
+struct RmsNormBwd : Function<RmsNormBwd> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& dy, double eps) {
+        ctx->save_for_backward({x, dy});
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        return {rmsnorm_bwd(x, dy, eps)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(3);
+        const variable_list s = ctx->get_saved_variables();
+        const double eps = ctx->saved_data["eps"].toDouble();
+        variable_list d = rmsnorm_bwd2(s[0], s[1], g[0], eps);
+        if (recorded({s[0], s[1], g[0]})) d = last(std::move(d));
+        d.emplace_back();
+        return d;
+    }
+};
+
+struct RmsNorm : Function<RmsNorm> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, double eps) {
+        ctx->save_for_backward({x});
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        return {rmsnorm(x, eps)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(2);
+        const Tensor x = ctx->get_saved_variables()[0];
+        return {RmsNormBwd::apply(x, g[0], ctx->saved_data["eps"].toDouble())[0], Tensor()};
+    }
+};
+
+Tensor swiglu_fwd(const Tensor& gu_) {
+    RECORD_FUNCTION("ebr_fused::block_swiglu", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(gu_.device());
+    const Tensor gu = dense(gu_);
+    std::vector<int64_t> shape = gu.sizes().vec();
+    shape.back() /= 2;
+    const Tensor y = at::empty(shape, gu.options());
+    const RowsOf r(gu);
+    check(ebr_block_swiglu(dtype_code(gu.scalar_type()), r.rows, (int)(r.width / 2), gu.data_ptr(), y.data_ptr(),
+                           stream_of(gu)),
+          "ebr_block_swiglu");
+    return y;
+}
+
+Tensor swiglu_bwd(const Tensor& gu_, const Tensor& dy_) {
+    RECORD_FUNCTION("ebr_fused::block_swiglu_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(gu_.device());
+    const Tensor gu = dense(gu_), dy = dense(dy_.to(gu_.scalar_type())), d = at::empty(gu.sizes(), gu.options());
+    const RowsOf r(gu);
+    check(ebr_block_swiglu_bwd(dtype_code(gu.scalar_type()), r.rows, (int)(r.width / 2), gu.data_ptr(), dy.data_ptr(),
+                               d.data_ptr(), stream_of(gu)),
+          "ebr_block_swiglu_bwd");
+    return d;
+}
+
+variable_list swiglu_bwd2(const Tensor& gu_, const Tensor& dy_, const Tensor& c_) {
+    RECORD_FUNCTION("ebr_fused::block_swiglu_bwd2", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(gu_.device());
+    const auto st = gu_.scalar_type();
+    const Tensor gu = dense(gu_), dy = dense(dy_.to(st)), c = dense(c_.to(st));
+    const Tensor ggu = at::empty(gu.sizes(), gu.options()), gdy = at::empty(dy.sizes(), dy.options());
+    const RowsOf r(gu);
+    check(ebr_block_swiglu_bwd2(dtype_code(st), r.rows, (int)(r.width / 2), gu.data_ptr(), dy.data_ptr(),
+                                c.data_ptr(), ggu.data_ptr(), gdy.data_ptr(), stream_of(gu)),
+          "ebr_block_swiglu_bwd2");
+    return {ggu, gdy};
+}
+
+struct SwiGLUBwd : Function<SwiGLUBwd> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& gu, const Tensor& dy) {
+        ctx->save_for_backward({gu, dy});
+        ctx->set_materialize_grads(false);
+        return {swiglu_bwd(gu, dy)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(2);
+        const variable_list s = ctx->get_saved_variables();
+        variable_list d = swiglu_bwd2(s[0], s[1], g[0]);
+        return recorded({s[0], s[1], g[0]}) ? last(std::move(d)) : d;
+    }
+};
+
+struct SwiGLU : Function<SwiGLU> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& gu) {
+        ctx->save_for_backward({gu});
+        ctx->set_materialize_grads(false);
+        return {swiglu_fwd(gu)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        if (!g[0].defined()) return variable_list(1);
+        return SwiGLUBwd::apply(ctx->get_saved_variables()[0], g[0]);
+    }
+};
+
+bool block_takes(const Tensor& x) {
+    return x.defined() && x.dim() >= 1 && x.numel() > 0 && dtype_code(x.scalar_type()) >= 0 &&
+           x.size(-1) < (int64_t(1) << 31) && plain_context();
+}
+
+py::object rms_norm(const py::handle& hx, double eps) {
+    const Tensor x = plain(hx);
+    if (!block_takes(x)) return py::none();
+    return py::cast(RmsNorm::apply(x, eps)[0]);
+}
+
+py::object swiglu(const py::handle& hgu) {
+    const Tensor gu = plain(hgu);
+    if (!block_takes(gu) || gu.size(-1) % 2) return py::none();
+    return py::cast(SwiGLU::apply(gu)[0]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Descent wrapper: first order only (the step size and the noise scale are constants of the schedule)
+// ---------------------------------------------------------------------------------------------------------------------
+
+void* vptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+Tensor noisy_bwd(const Tensor& z_, const Tensor& dv_, double eps) {
+    RECORD_FUNCTION("ebr_fused::descent_noisy_point_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(z_.device());
+    const Tensor z = dense(z_), dv = dense(dv_.to(z_.scalar_type())), dz = at::empty(z.sizes(), z.options());
+    check(ebr_descent_noisy_point_bwd(dtype_code(z.scalar_type()), (int)z.size(0), (int)z.size(1), (int)z.size(2),
+                                      (float)eps, z.data_ptr(), dv.data_ptr(), dz.data_ptr(), stream_of(z)),
+          "ebr_descent_noisy_point_bwd");
+    return dz;
+}
+
+variable_list step_bwd(const Tensor& v_, const Tensor& g_, const Tensor& alpha, const Tensor& active,
+                       const Tensor& rms, const Tensor& dout_, double eps) {
+    RECORD_FUNCTION("ebr_fused::descent_step_project_bwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(v_.device());
+    const auto st = v_.scalar_type();
+    const Tensor v = dense(v_), g = dense(g_.to(st)), dout = dense(dout_.to(st));
+    const Tensor dv = at::empty(v.sizes(), v.options()), dg = at::empty(v.sizes(), v.options());
+    const Tensor dz = active.defined() ? at::empty(v.sizes(), v.options()) : Tensor();
+    const int64_t B = v.size(0);
+    check(ebr_descent_step_project_bwd(dtype_code(st), (int)B, v.numel() / B, (float)eps, v.data_ptr(), g.data_ptr(),
+                                       fptr(alpha), static_cast<const uint8_t*>(vptr(active)), fptr(rms),
+                                       dout.data_ptr(), dv.data_ptr(), dg.data_ptr(), vptr(dz), stream_of(v)),
+          "ebr_descent_step_project_bwd");
+    return {dv, dg, dz};
+}
+
+struct NoisyPoint : Function<NoisyPoint> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& z_, const std::optional<Tensor>& noise_,
+                                 const std::optional<Tensor>& sigma_, double eps) {
+        const Tensor noise = noise_.value_or(Tensor()), sigma = sigma_.value_or(Tensor());
+        ctx->save_for_backward({z_});
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        RECORD_FUNCTION("ebr_fused::descent_noisy_point", std::vector<c10::IValue>());
+        const c10::DeviceGuard on(z_.device());
+        const Tensor z = dense(z_), v = at::empty(z.sizes(), z.options());
+        check(ebr_descent_noisy_point(dtype_code(z.scalar_type()), (int)z.size(0), (int)z.size(1), (int)z.size(2),
+                                      (float)eps, z.data_ptr(), vptr(noise), fptr(sigma), v.data_ptr(), stream_of(z)),
+              "ebr_descent_noisy_point");
+        return {v};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        variable_list out(4);
+        if (!g[0].defined()) return out;
+        const Tensor z = ctx->get_saved_variables()[0];
+        const double eps = ctx->saved_data["eps"].toDouble();
+        out[0] = noisy_bwd(z, g[0], eps);
+        if (recorded({z, g[0]})) out[0] = last({out[0]})[0];
+        return out;
+    }
+};
+
+struct StepProject : Function<StepProject> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& v_, const Tensor& g_, const Tensor& alpha,
+                                 const std::optional<Tensor>& z_, const std::optional<Tensor>& active_, double eps) {
+        const Tensor active = active_.value_or(Tensor());
+        RECORD_FUNCTION("ebr_fused::descent_step_project", std::vector<c10::IValue>());
+        const c10::DeviceGuard on(v_.device());
+        const auto st = v_.scalar_type();
+        const Tensor v = dense(v_), g = dense(g_.to(st)), z = z_ ? dense(z_->to(st)) : Tensor();
+        const int64_t B = v.size(0);
+        const Tensor out = at::empty(v.sizes(), v.options()), rms = at::empty({B}, v.options().dtype(at::kFloat));
+        check(ebr_descent_step_project(dtype_code(st), (int)B, v.numel() / B, (float)eps, v.data_ptr(), g.data_ptr(),
+                                       fptr(alpha), vptr(z), static_cast<const uint8_t*>(vptr(active)),
+                                       out.data_ptr(), static_cast<float*>(rms.data_ptr()), stream_of(v)),
+              "ebr_descent_step_project");
+        ctx->mark_non_differentiable({rms});
+        ctx->save_for_backward({v_, g_, alpha, active, rms});
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        return {out, rms};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& gr) {
+        variable_list out(6);
+        if (!gr[0].defined()) return out;
+        const variable_list s = ctx->get_saved_variables();
+        const double eps = ctx->saved_data["eps"].toDouble();
+        variable_list d = step_bwd(s[0], s[1], s[2], s[3], s[4], gr[0], eps);
+        if (recorded({s[0], s[1], gr[0]})) d = last(std::move(d));
+        out[0] = d[0];
+        out[1] = d[1];
+        out[3] = d[2];  // undefined without a mask: no row keeps z
+        return out;
+    }
+};
+
+// fp32 [rows] values of a per-row scalar: a Python float as given, a tensor of the data's dtype widened. Undefined for
+// what the Python layer has to look at (other dtypes and shapes, a schedule value that wants a gradient).
+Tensor per_row(const py::handle& x, const Tensor& like) {
+    const int64_t n = like.size(0);
+    if (py::isinstance<py::float_>(x) || py::isinstance<py::int_>(x))
+        return at::full({n}, x.cast<double>(), like.options().dtype(at::kFloat).requires_grad(false));
+    const Tensor t = plain(x);
+    if (!t.defined() || (t.requires_grad() && at::GradMode::is_enabled()) || !same_kind(t, like)) return {};
+    if (t.numel() != 1 && t.numel() != n) return {};
+    for (int64_t i = 1; i < t.dim(); ++i)
+        if (t.size(i) != 1) return {};
+    return t.detach().reshape(-1).expand({n}).to(at::kFloat).contiguous();
+}
+
+bool board(const Tensor& t) {
+    return t.defined() && t.dim() == 3 && t.numel() > 0 && dtype_code(t.scalar_type()) >= 0 &&
+           t.scalar_type() != at::kDouble && t.size(0) < (int64_t(1) << 31) && t.size(1) < (int64_t(1) << 31) &&
+           t.size(2) < (int64_t(1) << 31);
+}
+
+// rms_norm(z) + noise * sigma; ``hnoise`` None: rms_norm alone; ``hsigma`` None: the noise as it is.
+py::object noisy_point(const py::handle& hz, const py::handle& hnoise, const py::handle& hsigma, double eps) {
+    const Tensor z = plain(hz);
+    if (!board(z) || !plain_context()) return py::none();
+    Tensor noise, sigma;
+    if (!hnoise.is_none()) {
+        noise = plain(hnoise);
+        // noise that wants a gradient takes the Python node, which has the plain formula for it
+        if (!noise.defined() || noise.sizes() != z.sizes() || noise.device() != z.device() ||
+            (noise.requires_grad() && at::GradMode::is_enabled()))
+            return py::none();
+        noise = dense(noise.detach().to(z.scalar_type()));
+        if (!hsigma.is_none()) {
+            sigma = per_row(hsigma, z);
+            if (!sigma.defined()) return py::none();
+        }
+    }
+    return py::cast(NoisyPoint::apply(z, maybe(noise), maybe(sigma), eps)[0]);
+}
+
+py::object step_and_project(const py::handle& hv, const py::handle& hg, const py::handle& halpha,
+                            const py::handle& hz, const py::handle& hactive, double eps) {
+    const Tensor v = plain(hv), g = plain(hg), z = plain(hz);
+    if (!board(v) || !g.defined() || !z.defined() || !same_kind(v, g) || !same_kind(v, z) || !plain_context())
+        return py::none();
+    if (g.sizes() != v.sizes() || z.sizes() != v.sizes()) return py::none();
+    const Tensor alpha = per_row(halpha, v);
+    if (!alpha.defined()) return py::none();
+    Tensor active;
+    if (!hactive.is_none()) {
+        active = plain(hactive);
+        if (!active.defined() || active.numel() != v.size(0) || active.device() != v.device() ||
+            active.scalar_type() != at::kBool)
+            return py::none();
+        for (int64_t i = 1; i < active.dim(); ++i)
+            if (active.size(i) != 1) return py::none();
+        active = active.reshape(-1).contiguous().view(at::kByte);  // a bool is one byte, 0 or 1
+    }
+    return py::cast(StepProject::apply(v, g, alpha, active.defined() ? maybe(z) : std::nullopt, maybe(active), eps)[0]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Linear layers with split-K weight gradients (ebr_amd/linear.py states the rule and why)
+// ---------------------------------------------------------------------------------------------------------------------
+
+constexpr int64_t MIN_ROWS_PER_SPLIT = 1024;
+constexpr int64_t SPLIT8_OUTPUT = 1500000;
+
+int64_t splits(int64_t m, int64_t outputs) {
+    for (int64_t s = outputs >= SPLIT8_OUTPUT ? 8 : 16; s > 1; s /= 2)
+        if (m % s == 0 && m / s >= MIN_ROWS_PER_SPLIT) return s;
+    return 1;
+}
+
+// a^T b over the flattened leading dims.
+Tensor weight_grad(const Tensor& a, const Tensor& b) {
+    const Tensor a2 = a.reshape({-1, a.size(-1)}), b2 = b.reshape({-1, b.size(-1)});
+    if (recorded({a2, b2})) return at::matmul(a2.t(), b2);
+    const int64_t m = a2.size(0), n = a2.size(1), k = b2.size(1);
+    const int64_t s = a2.scalar_type() == at::kBFloat16 || a2.scalar_type() == at::kHalf ? splits(m, n * k) : 1;
+    if (s == 1) return at::matmul(a2.t(), b2);
+    const Tensor a3 = a2.contiguous().view({s, m / s, n}).transpose(1, 2);
+    const Tensor b3 = b2.contiguous().view({s, m / s, k});  // the right operand stays a contiguous batch
+    return at::bmm(a3, b3, at::kFloat).sum(0).to(a.scalar_type());
+}
+
+struct Linear;
+
+struct Dgrad : Function<Dgrad> {  // dX = dY W
+    static variable_list forward(AutogradContext* ctx, const Tensor& dy, const Tensor& w) {
+        ctx->save_for_backward({dy, w});
+        ctx->set_materialize_grads(false);
+        return {at::matmul(dy, w)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g);
+};
+
+struct Linear : Function<Linear> {  // Y = X W^T
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+        ctx->save_for_backward({x, w});
+        ctx->set_materialize_grads(false);
+        return {at::linear(x, w)};
+    }
+    // Gradients that the engine will not use are not computed.
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        variable_list out(2);
+        if (!g[0].defined()) return out;
+        const bool nx = ctx->needs_input_grad(0), nw = ctx->needs_input_grad(1);
+        const variable_list s = ctx->get_saved_variables();
+        if (nx) out[0] = Dgrad::apply(g[0], s[1])[0];
+        if (nw) out[1] = weight_grad(g[0], s[0]);
+        return out;
+    }
+};
+
+variable_list Dgrad::backward(AutogradContext* ctx, const variable_list& g) {
+    variable_list out(2);
+    if (!g[0].defined()) return out;
+    const bool ndy = ctx->needs_input_grad(0), nw = ctx->needs_input_grad(1);
+    const variable_list s = ctx->get_saved_variables();
+    if (ndy) out[0] = at::GradMode::is_enabled() ? Linear::apply(g[0], s[1])[0] : at::linear(g[0], s[1]);
+    if (nw) out[1] = weight_grad(s[0], g[0]);
+    return out;
+}
+
+py::object linear(const py::handle& hx, const py::handle& hw) {
+    const Tensor x = plain(hx), w = plain(hw);
+    if (!x.defined() || !w.defined() || x.dim() < 2 || w.dim() != 2 || x.size(-1) != w.size(1) || !same_kind(x, w) ||
+        x.numel() == 0 || w.numel() == 0 || !at::isFloatingType(x.scalar_type()) || !plain_context())
+        return py::none();
+    return py::cast(Linear::apply(x, w)[0]);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(ebr_host, m) {
+    if (ebr_attn_abi_version() != EBR_ATTN_ABI_VERSION)
+        throw std::runtime_error("libebr_attn.so has another ABI version than this module was built for");
+    m.def("attention", &attention);
+    m.def("rope_split", &rope_split);
+    m.def("rms_norm", &rms_norm);
+    m.def("swiglu", &swiglu);
+    m.def("noisy_point", &noisy_point);
+    m.def("step_and_project", &step_and_project);
+    m.def("linear", &linear);
+}

@@ -25,7 +25,7 @@ from typing import Optional, Tuple, Union
 import torch
 from torch.autograd.function import once_differentiable
 
-from ebr_amd import _capi
+from ebr_amd import _capi, _host
 from ebr_amd.fused_attn.loader import hip_library
 from ebr_amd.fused_attn.ops import _dtype_code, _stream
 
@@ -272,14 +272,26 @@ class _StepProject(torch.autograd.Function):
 # ---------------------------------------------------------------------------------------------------------------------
 
 
+def _native(name: str, *args):
+    """The native host path's result, or None for a call that it leaves to the nodes above."""
+    host = _host.module()
+    return None if host is None else getattr(host, name)(*args)
+
+
 def normalize(z: Tensor, eps: float = RMS_NORM_EPS) -> Tensor:
     """rms_norm over the last dim (reference EnergyDescent.normalize_descent_state, energy.py:287-288)."""
+    v = _native("noisy_point", z, None, None, eps)
+    if v is not None:
+        return v
     _check_board(z, "z")
     return _NoisyPoint.apply(z, None, None, None, eps)
 
 
 def noisy_point(z: Tensor, noise: Tensor, sigma: Scalar, eps: float = RMS_NORM_EPS) -> Tensor:
     """rms_norm(z) + noise * sigma (reference energy.py:226-227)."""
+    v = _native("noisy_point", z, noise, sigma, eps)
+    if v is not None:
+        return v
     _check_board(z, "z")
     if noise.shape != z.shape:
         raise ValueError(f"descent wrapper: noise {tuple(noise.shape)} != z {tuple(z.shape)}")
@@ -289,6 +301,9 @@ def noisy_point(z: Tensor, noise: Tensor, sigma: Scalar, eps: float = RMS_NORM_E
 
 def noisy_point_replayed(z: Tensor, noise: Tensor, eps: float = RMS_NORM_EPS) -> Tensor:
     """rms_norm(z) + noise (reference energy.py:230-232)."""
+    v = _native("noisy_point", z, noise, None, eps)
+    if v is not None:
+        return v
     _check_board(z, "z")
     if noise.shape != z.shape:
         raise ValueError(f"descent wrapper: noise {tuple(noise.shape)} != z {tuple(z.shape)}")
@@ -298,6 +313,9 @@ def noisy_point_replayed(z: Tensor, noise: Tensor, eps: float = RMS_NORM_EPS) ->
 def step_and_project(v: Tensor, grad: Tensor, alpha: Scalar, z: Tensor, active: Optional[Tensor],
                      eps: float = RMS_NORM_EPS) -> Tensor:
     """where(active, sphere(v - alpha * grad), z) (reference energy.py:235-241)."""
+    out = _native("step_and_project", v, grad, alpha, z, active, eps)
+    if out is not None:
+        return out
     _check_board(v, "v")
     if grad.shape != v.shape or z.shape != v.shape:
         raise ValueError(f"descent wrapper: grad {tuple(grad.shape)} / z {tuple(z.shape)} != v {tuple(v.shape)}")

@@ -23,7 +23,8 @@ kernels with 8-row tiles.
 
 Autograd: ``_FusedAttn`` (its backward is ``_FusedAttnBwd``) and ``_FusedAttnBwd`` (its backward is attn_bwd_bwd),
 both with ``setup_context`` as ``torch.func`` requires; ``fused_attention`` stays a single dynamo node through
-``allow_in_graph`` (reference ops.py:124-190).
+``allow_in_graph`` (reference ops.py:124-190). Plain GPU tensors outside tracing and transforms take the same nodes and
+launches natively (``ebr_amd._host``).
 """
 
 # No ``from __future__ import annotations``: custom_op schema inference needs real type objects.
@@ -34,7 +35,7 @@ import ctypes
 import torch
 import torch.nn.functional as F
 
-from ebr_amd import _capi
+from ebr_amd import _capi, _host
 from ebr_amd.fused_attn import dense
 from ebr_amd.fused_attn.loader import hip_library, mode
 
@@ -399,6 +400,12 @@ _fused_attention_apply = torch._dynamo.allow_in_graph(_fused_attention_apply)
 
 def fused_attention(q: Tensor, k: Tensor, v: Tensor, scale: Optional[float] = None) -> Tensor:
     """Non-causal softmax attention on [B, H, N, D], differentiable to second order."""
+    if not torch.compiler.is_compiling() and mode() != "reference":
+        host = _host.module()
+        if host is not None:
+            o = host.attention(q, k, v, None if scale is None else float(scale))
+            if o is not None:
+                return o
     return _fused_attention_apply(q, k, v, default_scale(q, scale))
 
 

@@ -21,6 +21,8 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from ebr_amd import _host
+
 Tensor = torch.Tensor
 
 SPLITS = (16, 8, 4, 2)
@@ -105,7 +107,10 @@ class _Linear(torch.autograd.Function):
 
 def linear(x: Tensor, w: Tensor, b: Optional[Tensor] = None) -> Tensor:
     """F.linear(x, w, b) with split-K weight gradients (the bias, if any, added by torch)."""
-    y = _Linear.apply(x, w)
+    host = None if torch.compiler.is_compiling() else _host.module()
+    y = None if host is None else host.linear(x, w)
+    if y is None:
+        y = _Linear.apply(x, w)
     return y if b is None else y + b
 
 

@@ -1,0 +1,250 @@
+"""The native host path (``ebr_amd._host``): it gives the Python nodes' bits for every derivative, and leaves to them
+every call that a mode, a transform, a hook or an argument check has to see."""
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from ebr_amd import _host, block, descent, linear
+from ebr_amd.fused_attn import fused_attention
+from ebr_amd.fused_attn.rope_split import rope_split
+from ebr_amd.layers import RotaryTable2D
+
+gpu = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _randn(shape, dtype, seed, device="cuda"):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(shape, generator=g).to(device=device, dtype=dtype)
+
+
+def _second_order(fn, xs, cots, seed=50):
+    """Outputs, gradients and the gradients' derivatives of ``fn`` for every input."""
+    xs = [x.detach().requires_grad_(True) for x in xs]
+    ys = fn(*xs)
+    ys = ys if isinstance(ys, tuple) else (ys,)
+    cots = [c.detach().requires_grad_(True) for c in cots]
+    first = torch.autograd.grad(ys, xs, cots, create_graph=True)
+    wrt = [*xs, *cots]
+    second = torch.autograd.grad(first, wrt, [_randn(t.shape, t.dtype, seed + i) for i, t in enumerate(first)],
+                                 allow_unused=True)
+    return [*ys, *first, *second]
+
+
+def _same(got, want):
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+            assert torch.equal(a, b)
+
+
+def _attn_inputs(dtype, shape, views, seed=0):
+    B, H, L, D = shape
+    if views == "qkv":
+        qkv = _randn((B, L, 3 * H * D), dtype, seed)
+        return [t.view(B, L, H, D).transpose(1, 2) for t in qkv.split(H * D, dim=-1)]
+    if views == "misaligned":  # rows that start 2 or 4 bytes past a 16-byte boundary: copied before the launch
+        return [_randn((B, H, L, D + 1), dtype, seed + i)[..., 1:] for i in range(3)]
+    return [_randn(shape, dtype, seed + i) for i in range(3)]
+
+
+CASES = [
+    ("attn", BF16, (2, 3, 17, 64), None), ("attn", F16, (1, 2, 130, 32), "qkv"), ("attn", F32, (2, 2, 33, 20), None),
+    ("attn", F32, (1, 2, 140, 64), "misaligned"), ("attn", BF16, (1, 2, 100, 128), "qkv"),
+    ("attn", BF16, (1, 1, 9, 200), None), ("rope", BF16, None, None), ("rope", F32, None, "scaled"),
+    ("norm", BF16, None, None), ("norm", torch.float64, None, None), ("swiglu", F16, None, "view"),
+    ("linear", BF16, None, None), ("linear", F32, None, "view"),
+]
+
+
+def _run(kind, dtype, shape, extra):
+    if kind == "attn":
+        cot = _randn(shape, dtype, 9)
+        return _second_order(lambda q, k, v: fused_attention(q, k, v, 0.2), _attn_inputs(dtype, shape, extra), [cot])
+    if kind == "rope":
+        rope = RotaryTable2D(16, 3, 5).cuda()
+        qs = torch.tensor([0.5, 2.0], device="cuda") if extra else None
+        return _second_order(lambda x: rope_split(x, *rope(), 2, qs), [_randn((4, 15, 96), dtype, 1)],
+                             [_randn((4, 2, 15, 16), dtype, 2 + i) for i in range(3)])
+    if kind == "norm":
+        return _second_order(lambda x: block.rms_norm(x, 1e-5), [_randn((3, 7, 24), dtype, 1)],
+                             [_randn((3, 7, 24), dtype, 2)])
+    if kind == "swiglu":
+        x = _randn((5, 2, 48), dtype, 1)
+        x = x.transpose(0, 1) if extra == "view" else x
+        return _second_order(block.swiglu, [x], [_randn((*x.shape[:-1], 24), dtype, 2)])
+    x = _randn((2, 1024, 32), dtype, 1)  # two split-K partials of 1,024 rows
+    x = x[:, ::2] if extra == "view" else x
+    return _second_order(linear.linear, [x, _randn((48, 32), dtype, 3)], [_randn((*x.shape[:-1], 48), dtype, 2)])
+
+
+@gpu
+@pytest.mark.parametrize("kind,dtype,shape,extra", CASES)
+def test_same_bits_as_the_python_nodes(monkeypatch, kind, dtype, shape, extra):
+    assert _host.module() is not None
+    got = _run(kind, dtype, shape, extra)
+    monkeypatch.setattr(_host, "module", lambda: None)
+    _same(got, _run(kind, dtype, shape, extra))
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("per_row,masked", [(True, True), (False, False), (True, False)])
+def test_descent_same_bits_as_the_python_nodes(monkeypatch, dtype, per_row, masked):
+    B, L, C = 3, 10, 64
+
+    def go():
+        z, n, g = (_randn((B, L, C), dtype, i).requires_grad_(i != 1) for i in range(3))
+        sig = torch.tensor([0.1, 0.2, 0.3], device="cuda").to(dtype).view(B, 1, 1) if per_row else 0.25
+        act = torch.tensor([True, False, True], device="cuda").view(B, 1, 1) if masked else None
+        vs = [descent.noisy_point(z, n, sig), descent.noisy_point_replayed(z, n), descent.normalize(z)]
+        outs = [descent.step_and_project(v, g, sig, z, act) for v in vs]
+        return [*vs, *outs, *torch.autograd.grad(outs, (z, g), [_randn((B, L, C), dtype, 7 + i) for i in range(3)])]
+
+    got = go()
+    monkeypatch.setattr(_host, "module", lambda: None)
+    _same(got, go())
+
+
+@gpu
+def test_a_single_used_gradient_and_unused_outputs(monkeypatch):
+    """Zero rows for the cotangents nobody gives, in attention and in the rotary split."""
+    rope = RotaryTable2D(16, 3, 5).cuda()
+
+    def go():
+        x = _randn((2, 15, 96), BF16, 1).requires_grad_(True)
+        q, k, v = rope_split(x, *rope(), 2)
+        o = fused_attention(q, k, v)
+        (dq,) = torch.autograd.grad(o, q, _randn(o.shape, BF16, 2), create_graph=True)
+        return [*torch.autograd.grad(dq, x, _randn(dq.shape, BF16, 3), retain_graph=True),
+                *torch.autograd.grad(k, x, _randn(k.shape, BF16, 4))]
+
+    got = go()
+    monkeypatch.setattr(_host, "module", lambda: None)
+    _same(got, go())
+
+
+@gpu
+def test_plain_calls_take_it():
+    q = _randn((1, 2, 16, 16), BF16, 0).requires_grad_(True)
+    x = _randn((1, 4, 24), BF16, 0).requires_grad_(True)
+    rope = RotaryTable2D(4, 2, 2).cuda()
+    for y in (fused_attention(q, q, q), block.rms_norm(q, 1e-5), block.swiglu(q), linear.linear(q, q[0, 0]),
+              descent.normalize(q[0]), descent.step_and_project(q[0], q[0], 0.1, q[0], None),
+              rope_split(x, *rope(), 2)[0]):
+        assert "CppNode" in y.grad_fn.name()
+
+
+@gpu
+def test_no_derivative_past_the_second():
+    x = _randn((4, 16), F32, 0).requires_grad_(True)
+    (g,) = torch.autograd.grad(block.rms_norm(x, 1e-5).square().sum(), x, create_graph=True)
+    (h,) = torch.autograd.grad(g.square().sum(), x, create_graph=True)
+    with pytest.raises(RuntimeError):
+        h.sum().backward()
+    q, k, v = (_randn((1, 1, 8, 16), F32, i).requires_grad_(True) for i in range(3))
+    (g,) = torch.autograd.grad(fused_attention(q, k, v).square().sum(), q, create_graph=True)
+    (h,) = torch.autograd.grad(g.square().sum(), q, create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(h.sum(), q)
+
+
+class _Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.ops = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.ops.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@gpu
+def test_modes_transforms_and_hooks_see_the_ops():
+    q, k, v = (_randn((1, 2, 9, 16), F32, i).requires_grad_(True) for i in range(3))
+    with _Seen() as seen:
+        want = fused_attention(q, k, v)
+    assert "ebr_fused.attn_fwd.default" in seen.ops
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t, lambda t: t):
+        o = fused_attention(q, k, v)
+    assert len(packed) == 5 and torch.equal(o, want)
+    g = torch.func.grad(lambda x: fused_attention(x, k.detach(), v.detach()).sum())(q.detach())
+    assert torch.equal(g, torch.autograd.grad(want.sum(), q)[0])
+    out = torch.compile(lambda x: fused_attention(x, k, v) * 2, backend="aot_eager", fullgraph=True)(q)
+    assert torch.equal(out, want * 2)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        torch.func.jvp(lambda x: fused_attention(x, k.detach(), v.detach()), (q.detach(),), (q.detach(),))
+
+
+@gpu
+def test_refused_calls_stay_refused():
+    q = _randn((1, 2, 9, 16), F32, 0)
+    with pytest.raises(ValueError):
+        fused_attention(q, q[:, :1], q)
+    with pytest.raises(ValueError):
+        fused_attention(q, q.half(), q)
+    with pytest.raises(ValueError):
+        fused_attention(*[_randn((1, 1, 4, 264), F32, 0)] * 3)
+    with pytest.raises(ValueError):
+        block.swiglu(_randn((3, 5), F32, 0))
+    with pytest.raises(TypeError):
+        descent.noisy_point(_randn((2, 3, 4), BF16, 0), _randn((2, 3, 4), BF16, 0), torch.ones((2, 1, 1)).cuda())
+    with pytest.raises(ValueError):
+        descent.step_and_project(*[_randn((2, 3, 4), F32, 0)] * 2, torch.ones((3, 1, 1)).cuda(),
+                                 _randn((2, 3, 4), F32, 0), None)
+    assert fused_attention(*[_randn((1, 2, 9, 20), BF16, 0)] * 3).shape == (1, 2, 9, 20)  # padded in Python
+    assert fused_attention(*[_randn((0, 2, 9, 16), BF16, 0)] * 3).shape == (0, 2, 9, 16)
+
+
+@gpu
+def test_on_a_side_stream_and_from_threads():
+    import threading
+
+    q, k, v = (_randn((4, 2, 40, 64), BF16, i) for i in range(3))
+    want = fused_attention(q, k, v)
+    got = [None] * 4
+    torch.cuda.synchronize()
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            x = q.clone().requires_grad_(True)
+            o = fused_attention(x, k, v)
+            (g,) = torch.autograd.grad(o, x, v)
+        s.synchronize()
+        got[i] = (o.detach(), g)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for o, g in got:
+        assert torch.equal(o, want) and torch.equal(g, got[0][1])
+
+
+def test_leaves_other_tensors_to_python():
+    host = _host.module()
+    if host is None:
+        pytest.skip("the native host path is not built")
+    x = torch.randn(2, 4, 8, 16)
+    assert host.attention(x, x, x, None) is None and host.attention(1, None, "x", 0.5) is None
+    assert host.rms_norm(x, 1e-5) is None and host.swiglu(x) is None and host.linear(x, x[0, 0]) is None
+    assert host.noisy_point(x[0], x[0], 0.1, 1e-5) is None
+    assert host.step_and_project(x[0], x[0], 0.1, x[0], None, 1e-5) is None
+    assert host.rope_split(x[0], x[0, 0], x[0, 0], 2, None) is None
+    with FakeTensorMode():
+        f = torch.empty(2, 4, 8, 16, device="cuda")
+        assert host.attention(f, f, f, None) is None and host.rms_norm(f, 1e-5) is None
+
+
+def test_host_command_links_the_library_beside_it():
+    from pathlib import Path
+
+    from ebr_amd import build
+
+    cmd = build.host_command(Path("x.so"))
+    assert "-lebr_attn" in cmd and "-Wl,-rpath,$ORIGIN" in cmd and cmd[-1] == "x.so"
