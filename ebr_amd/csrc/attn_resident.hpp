@@ -12,30 +12,7 @@
 //                              slot order of the accumulator-derived B operand (attn_tiles.hpp).
 // So no transposed copy of any input exists, and the chunk loops run without barriers.
 
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-#define EBR_LDS __attribute__((address_space(3)))
-
 constexpr uint32_t BUF_RSRC_WORD3 = 0x00020000;  // raw buffer, dword data format (gfx9 family)
-
-template <int DP> struct Sw {
-    static constexpr int NCK = DP / 8;   // 16-byte chunks per row
-    static constexpr int ROWB = DP * 2;  // bytes per row
-    static constexpr int RPI = 64 / NCK; // rows moved by one 64-lane x 16-byte load
-    // Depends on x mod 16 only, so every 16-row tile (and every 32-row chunk) has the same per-lane pattern.
-    static __device__ __forceinline__ int swz(int x) {
-        if constexpr (DP == 32) {
-            return (x >> 2) & 3;
-        } else if constexpr (DP == 64) {
-            // bits 1 and 2 of x swapped: with 4 or more waves per CU, the A-operand reads of 16 rows x 2 chunk
-            // positions then meet no bank conflict (measured with SQ_LDS_BANK_CONFLICT; the earlier
-            // (x & 7) ^ (x >> 3 & 1) cost a quarter of the read cycles), and the transposed reads stay conflict-free
-            return (x & 1) | ((x & 4) >> 1) | ((x & 2) << 1);
-        } else {
-            return x & 15;
-        }
-    }
-    static __device__ __forceinline__ int off(int x, int c) { return x * ROWB + 16 * (c ^ swz(x)); }
-};
 
 // Per-lane byte offsets inside a 16-row tile (a) and a 32-row chunk (tr), fixed for the whole kernel.
 template <typename T, int DP> struct LaneOff {

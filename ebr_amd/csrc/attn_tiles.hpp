@@ -24,6 +24,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ebr {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -40,10 +42,35 @@ constexpr int STAT_MAX = 128;               // longest L handled by the one-work
 constexpr int DMAX_WIDE = 256;              // widest head dim, 16-bit and fp32 (above 128: the streamed kernels)
 constexpr int DMAX_F64 = 256;               // widest head dim of the fp64 kernels
 
+// fp32 inputs come as one of three types of the same memory layout:
+//   float  v_mfma_f32_16x16x4_f32 on fp32 chunks in LDS, natural and transposed;
+//   f32s   each value split into three bf16 planes (below), on the bf16 MFMA;
+//   f32n   v_mfma_f32_16x16x4_f32 on natural chunks alone (half the LDS): what an f32s kernel falls back to.
+struct f32s {
+    float v;
+};
+struct f32n {
+    float v;
+    __device__ operator float() const { return v; }
+};
+
+// Split products. x = hi + mid + lo with each part x's remainder rounded to bf16 (8 significant bits each), which is
+// exact for a 24-bit significand; |mid| <= 2^-8 |x|, |lo| <= 2^-16 |x|. A product of two values is the six products of
+// parts down to 2^-16 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three left out are below 2^-23 of it
+// at worst and 2^-27 in the mean, of either sign. Each product of parts is exact in the MFMA's fp32, and the small
+// ones enter an accumulator first. Six bf16 MFMAs of k = 32 take 96 cycles where eight fp32 MFMAs of k = 4 take 256,
+// and a plane is read transposed, so a tensor is staged once instead of natural and transposed. Measured at B H = 64,
+// L = 400, D = 64 (fp32 MFMA -> split): forward 41.4 -> 31.9, backward 126 -> 85, bwd_bwd 328 -> 186 us, the error
+// against 64 bits 4.6e-7 -> 3.6e-7, 5.9e-7 -> 5.0e-7, 7.2e-7 -> 6.1e-7 (fewer roundings per sum).
+// Non-finite inputs (and values past bf16's range) do not survive the split: they give NaN wherever they enter, and a
+// workgroup whose outputs hold a NaN computes them again with f32n (see redo_if_nan), so the results for such inputs
+// are those of plain fp32 arithmetic.
+constexpr int NPLANE = 3;
+
 template <typename T> struct ET;
 
 template <> struct ET<__bf16> {
-    static constexpr bool F32 = false;
+    static constexpr bool F32 = false, SPLIT = false, WIDE = false;
     static constexpr int VEC = 8;           // elements per 16-byte vector
     static constexpr int PADN = 8;          // natural layout row padding (elements)
     static constexpr int PADT = 8;          // transposed layout row padding (elements)
@@ -62,7 +89,7 @@ template <> struct ET<__bf16> {
 };
 
 template <> struct ET<_Float16> {
-    static constexpr bool F32 = false;
+    static constexpr bool F32 = false, SPLIT = false, WIDE = false;
     static constexpr int VEC = 8;
     static constexpr int PADN = 8;
     static constexpr int PADT = 8;
@@ -78,11 +105,43 @@ template <> struct ET<_Float16> {
 };
 
 template <> struct ET<float> {
-    static constexpr bool F32 = true;
+    static constexpr bool F32 = true, SPLIT = false, WIDE = true;  // fp32 MFMA; split planes; 4 bytes in memory
     static constexpr int VEC = 4;
     static constexpr int PADN = 4;
     static constexpr int PADT = 4;
 };
+
+template <> struct ET<f32n> : ET<float> {};
+
+template <> struct ET<f32s> {
+    static constexpr bool F32 = false, SPLIT = true, WIDE = true;
+    static constexpr int VEC = 4;
+};
+
+// 16-byte chunks of a 16-bit row of DP elements, XOR-swizzled by the row so that the reads of a 16-row tile meet no
+// bank conflict.
+template <int DP> struct Sw {
+    static constexpr int NCK = DP / 8;   // 16-byte chunks per row
+    static constexpr int ROWB = DP * 2;  // bytes per row
+    static constexpr int RPI = 64 / NCK; // rows moved by one 64-lane x 16-byte load
+    // Depends on x mod 16 only, so every 16-row tile (and every 32-row chunk) has the same per-lane pattern.
+    static __device__ __forceinline__ int swz(int x) {
+        if constexpr (DP == 32) {
+            return (x >> 2) & 3;
+        } else if constexpr (DP == 64) {
+            // bits 1 and 2 of x swapped: with 4 or more waves per CU, the A-operand reads of 16 rows x 2 chunk
+            // positions then meet no bank conflict (measured with SQ_LDS_BANK_CONFLICT; the earlier
+            // (x & 7) ^ (x >> 3 & 1) cost a quarter of the read cycles), and the transposed reads stay conflict-free
+            return (x & 1) | ((x & 4) >> 1) | ((x & 2) << 1);
+        } else {
+            return x & 15;
+        }
+    }
+    static __device__ __forceinline__ int off(int x, int c) { return x * ROWB + 16 * (c ^ swz(x)); }
+};
+
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+#define EBR_LDS __attribute__((address_space(3)))
 
 // Layout constants of one (T, DP) instantiation. DP is the head dimension padded to the d-chunk width.
 template <typename T, int DP> struct Lay {
@@ -96,11 +155,50 @@ template <typename T, int DP> struct Lay {
     // fp32 above DP = 128: a transposed copy of each chunk does not fit beside the natural one (the backward of the
     // backward stages four tensors), so seq-contractions read their A operand from the natural rows, one element per
     // k slot, and a tensor wanted in both layouts is staged once.
-    static constexpr bool NATSEQ = ET<T>::F32 && DP > 128;
+    static constexpr bool NATSEQ = ET<T>::F32 && (DP > 128 || std::is_same_v<T, f32n>);
     static constexpr int TRB = NATSEQ ? 0 : DP * PT * (int)sizeof(T);  // bytes of one transposed chunk
     static_assert(DP % CW == 0, "DP must be a multiple of the d-chunk width");
     static_assert(NATB % 16 == 0 && TRB % 16 == 0, "LDS regions must stay 16-byte aligned");
 };
+
+// Split planes: plane i of a chunk holds its 32 rows as bf16 in the swizzled natural layout; seq-contractions read them
+// transposed (ds_read_b64_tr_b16), so a tensor is staged once.
+template <int DP> struct Lay<f32s, DP> {
+    static constexpr int VEC = 4;
+    static constexpr int CW = 32;
+    static constexpr int NC = DP / CW;
+    static constexpr int NT = DP / 16;
+    static constexpr int PLANE = CH * Sw<DP>::ROWB;  // bytes of one plane of a chunk
+    static constexpr int PN = DP / 2;                // plane row pitch in 4-byte units (the tile pointers' type)
+    static constexpr int NATB = NPLANE * PLANE;
+    static constexpr bool NATSEQ = true;
+    static constexpr int TRB = 0;
+};
+
+// Eight values as three planes of packed bf16.
+__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u32x4 (&out)[NPLANE]) {
+    float r[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+    for (int i = 0; i < NPLANE; ++i) {
+        bf16x8 h;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            h[e] = (__bf16)r[e];
+            r[e] -= (float)h[e];  // exact
+        }
+        out[i] = __builtin_bit_cast(u32x4, h);
+    }
+}
+
+// acc += sum over the six products of parts, the small ones first.
+__device__ __forceinline__ f32x4 mma_split(const u32x4 (&a)[NPLANE], const u32x4 (&b)[NPLANE], f32x4 acc) {
+    acc = ET<__bf16>::mma(a[2], b[0], acc);
+    acc = ET<__bf16>::mma(a[0], b[2], acc);
+    acc = ET<__bf16>::mma(a[1], b[1], acc);
+    acc = ET<__bf16>::mma(a[1], b[0], acc);
+    acc = ET<__bf16>::mma(a[0], b[1], acc);
+    return ET<__bf16>::mma(a[0], b[0], acc);
+}
 
 // Column of chunk-local row x in the transposed LDS layout (see the header comment).
 template <typename T> __device__ __forceinline__ int tr_col(int x) {
@@ -173,19 +271,39 @@ template <typename T, int DP> struct OwnFrag {
     u32x4 v[Lay<T, DP>::NC];
 };
 
+template <int DP> struct OwnFrag<f32s, DP> {
+    u32x4 v[Lay<f32s, DP>::NC][NPLANE];
+};
+
 template <typename T, int DP>
 __device__ __forceinline__ void load_own(OwnFrag<T, DP>& f, const T* base, int64_t srow, int row, int L, int D,
                                          int g) {
     using LY = Lay<T, DP>;
-    // Unconditional loads from a clamped (always valid) address, then a select: no branch, so the loads of several
-    // fragments stay in flight together.
-    const T* p = base + (int64_t)(row < L ? row : L - 1) * srow;
+    if constexpr (ET<T>::SPLIT) {
+        const T* p = base + (int64_t)(row < L ? row : L - 1) * srow;
+        f32x4 x[LY::NC][2];
 #pragma unroll
-    for (int c = 0; c < LY::NC; ++c) {
-        const int d0 = c * LY::CW + g * LY::VEC;
-        const u32x4 z = {0u, 0u, 0u, 0u};
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p + (d0 < D ? d0 : D - LY::VEC));
-        f.v[c] = (row < L && d0 < D) ? v : z;
+        for (int c = 0; c < LY::NC; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int d0 = c * LY::CW + 8 * g + 4 * h;
+                const f32x4 v = *reinterpret_cast<const f32x4*>(p + (d0 < D ? d0 : D - LY::VEC));
+                x[c][h] = (row < L && d0 < D) ? v : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+        for (int c = 0; c < LY::NC; ++c) split8(x[c][0], x[c][1], f.v[c]);
+        return;
+    } else {
+        // Unconditional loads from a clamped (always valid) address, then a select: no branch, so the loads of several
+        // fragments stay in flight together.
+        const T* p = base + (int64_t)(row < L ? row : L - 1) * srow;
+#pragma unroll
+        for (int c = 0; c < LY::NC; ++c) {
+            const int d0 = c * LY::CW + g * LY::VEC;
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            const u32x4 v = *reinterpret_cast<const u32x4*>(p + (d0 < D ? d0 : D - LY::VEC));
+            f.v[c] = (row < L && d0 < D) ? v : z;
+        }
     }
 }
 
@@ -195,7 +313,20 @@ __device__ __forceinline__ float frag_dot(const OwnFrag<T, DP>& a, const OwnFrag
     float s = 0.f;
 #pragma unroll
     for (int c = 0; c < Lay<T, DP>::NC; ++c) {
-        if constexpr (ET<T>::F32) {
+        if constexpr (ET<T>::SPLIT) {
+            float x[8] = {}, y[8] = {};
+#pragma unroll
+            for (int i = NPLANE - 1; i >= 0; --i) {  // the parts' sum is the value
+                const bf16x8 p = __builtin_bit_cast(bf16x8, a.v[c][i]), q = __builtin_bit_cast(bf16x8, b.v[c][i]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    x[e] += (float)p[e];
+                    y[e] += (float)q[e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += x[e] * y[e];
+        } else if constexpr (ET<T>::F32) {
             const f32x4 x = __builtin_bit_cast(f32x4, a.v[c]);
             const f32x4 y = __builtin_bit_cast(f32x4, b.v[c]);
             s += x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3];
@@ -217,17 +348,29 @@ __device__ __forceinline__ float frag_dot(const OwnFrag<T, DP>& a, const OwnFrag
 template <typename T, int DP>
 __device__ __forceinline__ void mma_d(f32x4& acc, const T* Xn_tile, const OwnFrag<T, DP>& f, int l16, int g) {
     using LY = Lay<T, DP>;
-    const T* p = Xn_tile + l16 * LY::PN + g * LY::VEC;
+    if constexpr (ET<T>::SPLIT) {
+        const unsigned char* base = reinterpret_cast<const unsigned char*>(Xn_tile);
 #pragma unroll
-    for (int c = 0; c < LY::NC; ++c) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(p + c * LY::CW);
-        if constexpr (ET<T>::F32) {
-            const f32x4 af = __builtin_bit_cast(f32x4, a);
-            const f32x4 bf = __builtin_bit_cast(f32x4, f.v[c]);
+        for (int c = 0; c < LY::NC; ++c) {
+            u32x4 x[NPLANE];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], bf[e], acc, 0, 0, 0);
-        } else {
-            acc = ET<T>::mma(a, f.v[c], acc);
+            for (int i = 0; i < NPLANE; ++i)
+                x[i] = *reinterpret_cast<const u32x4*>(base + i * LY::PLANE + Sw<DP>::off(l16, 4 * c + g));
+            acc = mma_split(x, f.v[c], acc);
+        }
+    } else {
+        const T* p = Xn_tile + l16 * LY::PN + g * LY::VEC;
+#pragma unroll
+        for (int c = 0; c < LY::NC; ++c) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(p + c * LY::CW);
+            if constexpr (ET<T>::F32) {
+                const f32x4 af = __builtin_bit_cast(f32x4, a);
+                const f32x4 bf = __builtin_bit_cast(f32x4, f.v[c]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], bf[e], acc, 0, 0, 0);
+            } else {
+                acc = ET<T>::mma(a, f.v[c], acc);
+            }
         }
     }
 }
@@ -243,10 +386,16 @@ template <typename T> struct SeqB {
 template <> struct SeqB<float> {
     f32x4 h0, h1;
 };
+template <> struct SeqB<f32n> : SeqB<float> {};
+template <> struct SeqB<f32s> {
+    u32x4 v[NPLANE];
+};
 
 template <typename T> __device__ __forceinline__ SeqB<T> make_seqb(f32x4 p0, f32x4 p1) {
     SeqB<T> b;
-    if constexpr (ET<T>::F32) {
+    if constexpr (ET<T>::SPLIT) {
+        split8(p0, p1, b.v);
+    } else if constexpr (ET<T>::F32) {
         b.h0 = p0;
         b.h1 = p1;
     } else {
@@ -289,32 +438,53 @@ template <typename T> struct SeqA {
 template <> struct SeqA<float> {
     f32x4 h0, h1;
 };
+template <> struct SeqA<f32n> : SeqA<float> {};
+template <> struct SeqA<f32s> {
+    u32x4 v[NPLANE];
+};
 
 // A operand of d tile t: lane (d = 16 t + l16, group g). Under NATSEQ, Xt holds the chunk's natural rows.
 template <typename T, int DP> __device__ __forceinline__ SeqA<T> read_seqa(const T* Xt, int t, int l16, int g) {
     using LY = Lay<T, DP>;
     SeqA<T> a;
-    if constexpr (LY::NATSEQ) {
-        const T* q = Xt + 16 * t + l16;
+    if constexpr (ET<T>::SPLIT) {
+        const int k = l16 >> 2, d = 16 * t + 4 * (l16 & 3);
+        const unsigned char* p =
+            reinterpret_cast<const unsigned char*>(Xt) + Sw<DP>::off(4 * g + k, d >> 3) + (d & 7) * 2;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            a.h0[r] = q[(4 * g + r) * LY::PN];
-            a.h1[r] = q[(16 + 4 * g + r) * LY::PN];
+        for (int i = 0; i < NPLANE; ++i) {
+            const unsigned char* q = p + i * LY::PLANE;
+            const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((EBR_LDS s16x4*)q));
+            const u32x2 hi = __builtin_bit_cast(
+                u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((EBR_LDS s16x4*)(q + 16 * Sw<DP>::ROWB)));
+            a.v[i] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+        return a;
+    } else {
+        if constexpr (LY::NATSEQ) {
+            const T* q = Xt + 16 * t + l16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                a.h0[r] = q[(4 * g + r) * LY::PN];
+                a.h1[r] = q[(16 + 4 * g + r) * LY::PN];
+            }
+            return a;
+        }
+        const T* p = Xt + (16 * t + l16) * LY::PT;
+        if constexpr (ET<T>::F32) {
+            a.h0 = *reinterpret_cast<const f32x4*>(p + 4 * g);
+            a.h1 = *reinterpret_cast<const f32x4*>(p + 16 + 4 * g);
+        } else {
+            a.v = *reinterpret_cast<const u32x4*>(p + 8 * g);
         }
         return a;
     }
-    const T* p = Xt + (16 * t + l16) * LY::PT;
-    if constexpr (ET<T>::F32) {
-        a.h0 = *reinterpret_cast<const f32x4*>(p + 4 * g);
-        a.h1 = *reinterpret_cast<const f32x4*>(p + 16 + 4 * g);
-    } else {
-        a.v = *reinterpret_cast<const u32x4*>(p + 8 * g);
-    }
-    return a;
 }
 
 template <typename T> __device__ __forceinline__ f32x4 mma_seq(f32x4 acc, const SeqA<T>& a, const SeqB<T>& b) {
-    if constexpr (ET<T>::F32) {
+    if constexpr (ET<T>::SPLIT) {
+        return mma_split(a.v, b.v, acc);
+    } else if constexpr (ET<T>::F32) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.h0[r], b.h0[r], acc, 0, 0, 0);
 #pragma unroll
@@ -345,12 +515,16 @@ template <typename T, int DP, int N> struct Stage {
     static constexpr int ITEMS = (TOTAL + MIN_THREADS - 1) / MIN_THREADS;
     u32x4 r[N][ITEMS];
 
+    // Consecutive lanes take consecutive rows where a transposed copy is written (no bank conflicts there), else
+    // consecutive vectors of a row (whole rows per load).
+    static __device__ __forceinline__ int row_of(int it) { return ET<T>::SPLIT ? it / VPR : it % CH; }
+    static __device__ __forceinline__ int vec_of(int it) { return ET<T>::SPLIT ? it % VPR : it / CH; }
+
     __device__ __forceinline__ void load(const Src<T, N>& s, int x0, int L, int D, int tid, int nthr) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const int it = tid + i * nthr;
-            const int x = it % CH;  // consecutive lanes take consecutive rows (conflict-free transposed writes)
-            const int c = it / CH;
+            const int x = row_of(it), c = vec_of(it);
             const int row = x0 + x;
             const int d0 = c * LY::VEC;
             const bool ok = it < TOTAL && row < L && d0 < D;
@@ -372,26 +546,45 @@ template <typename T, int DP, int N> struct Stage {
         for (int i = 0; i < ITEMS; ++i) {
             const int it = tid + i * nthr;
             if (it >= TOTAL) continue;
-            const int x = it % CH;
-            const int c = it / CH;
+            const int x = row_of(it), c = vec_of(it);
             const int d0 = c * LY::VEC;
-            const int col = tr_col<T>(x);
+            if constexpr (ET<T>::SPLIT) {
+                const int off = Sw<DP>::off(x, d0 >> 3) + (d0 & 7) * 2;
 #pragma unroll
-            for (int t = 0; t < N; ++t) {
-                if (Xn[t]) *reinterpret_cast<u32x4*>(Xn[t] + x * LY::PN + d0) = r[t][i];
-                if constexpr (LY::NATSEQ) {
-                    if (Xt[t] && Xt[t] != Xn[t]) *reinterpret_cast<u32x4*>(Xt[t] + x * LY::PN + d0) = r[t][i];
-                } else if (Xt[t]) {
-                    T* p = Xt[t] + d0 * LY::PT + col;
-                    if constexpr (ET<T>::F32) {
-                        const f32x4 e = __builtin_bit_cast(f32x4, r[t][i]);
+                for (int t = 0; t < N; ++t) {
+                    unsigned char* p = reinterpret_cast<unsigned char*>(Xn[t] ? Xn[t] : Xt[t]) + off;
+                    f32x4 e = __builtin_bit_cast(f32x4, r[t][i]);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) p[j * LY::PT] = e[j];
-                    } else {
-                        using V8 = typename ET<T>::v8;
-                        const V8 e = __builtin_bit_cast(V8, r[t][i]);
+                    for (int k = 0; k < NPLANE; ++k) {
+                        bf16x4 h;
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) p[j * LY::PT] = e[j];
+                        for (int j = 0; j < 4; ++j) {
+                            h[j] = (__bf16)e[j];
+                            e[j] -= (float)h[j];
+                        }
+                        *reinterpret_cast<u32x2*>(p + k * LY::PLANE) = __builtin_bit_cast(u32x2, h);
+                    }
+                }
+                continue;
+            } else {
+                const int col = tr_col<T>(x);
+#pragma unroll
+                for (int t = 0; t < N; ++t) {
+                    if (Xn[t]) *reinterpret_cast<u32x4*>(Xn[t] + x * LY::PN + d0) = r[t][i];
+                    if constexpr (LY::NATSEQ) {
+                        if (Xt[t] && Xt[t] != Xn[t]) *reinterpret_cast<u32x4*>(Xt[t] + x * LY::PN + d0) = r[t][i];
+                    } else if (Xt[t]) {
+                        T* p = Xt[t] + d0 * LY::PT + col;
+                        if constexpr (ET<T>::F32) {
+                            const f32x4 e = __builtin_bit_cast(f32x4, r[t][i]);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) p[j * LY::PT] = e[j];
+                        } else {
+                            using V8 = typename ET<T>::v8;
+                            const V8 e = __builtin_bit_cast(V8, r[t][i]);
+#pragma unroll
+                            for (int j = 0; j < 8; ++j) p[j * LY::PT] = e[j];
+                        }
                     }
                 }
             }
@@ -428,7 +621,7 @@ template <int NS> struct StatStage {
 // ---------------------------------------------------------------------------------------------------------------------
 
 template <typename T> __device__ __forceinline__ void store4(T* p, f32x4 v) {
-    if constexpr (ET<T>::F32) {
+    if constexpr (ET<T>::WIDE) {
         *reinterpret_cast<f32x4*>(p) = v;
     } else {
         using V4 = typename ET<T>::v4;
@@ -453,7 +646,7 @@ template <typename T> __device__ __forceinline__ u32x2 pack4(f32x4 v) {
 }
 
 template <typename T> __device__ __forceinline__ f32x4 load4(const T* p) {
-    if constexpr (ET<T>::F32) {
+    if constexpr (ET<T>::WIDE) {
         return *reinterpret_cast<const f32x4*>(p);
     } else {
         using V4 = typename ET<T>::v4;

@@ -103,12 +103,41 @@ __device__ __forceinline__ void store_rows(void* out, int64_t row_off, const f32
 // Forward (row pass): online softmax over 32-key chunks.
 // =====================================================================================================================
 
-// Wider rows than DP = 128 run 256-thread workgroups (one wave per SIMD, every register for the wave).
-template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512) void k_fwd(Args a) {
+// Whether a lane's sums hold a NaN (infinities of both signs count as one).
+template <int N> __device__ __forceinline__ float total(const f32x4 (&v)[N]) {
+    float s = 0.f;
+#pragma unroll
+    for (int t = 0; t < N; ++t) s += (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
+    return s;
+}
+
+// Runs ``body`` (which returns whether an output row of this lane holds a NaN) with T; split products give NaN for
+// non-finite inputs where fp32 arithmetic may give an infinity, so a workgroup that saw a NaN runs again with f32n,
+// which overwrites everything the first run wrote.
+template <typename T, class Body> __device__ __forceinline__ void redo_if_nan(Body&& body) {
+    const bool bad = body(T{});
+    if constexpr (ET<T>::SPLIT) {
+        if (__syncthreads_or(bad)) body(f32n{});
+    }
+}
+
+// The next chunk's loads start under the computation of a chunk, or, in the split backward kernels, after it, so that
+// it has their registers (bwd_bwd 206 -> 189 us at 64 slices, L = 400, D = 64: fewer spills weigh more than the loads'
+// latency, which the other workgroup of the CU covers).
+template <typename T> constexpr bool loads_after() { return ET<T>::SPLIT; }
+
+template <typename T, int DP> struct FwdSmem {
+    static constexpr int ONE = Lay<T, DP>::NATB + (Lay<T, DP>::NATSEQ ? Lay<T, DP>::NATB : Lay<T, DP>::TRB);
+    // The split forward up to D = 64 writes a chunk while the one before is read: one barrier per chunk instead of two
+    // (33.2 -> 31.9 us at 64 slices, L = 400, D = 64; the backward gained nothing from it, and at D = 128 two buffers
+    // leave a CU one workgroup: 94 against 67 us at 512 slices, L = 129).
+    static constexpr bool TWICE = ET<T>::SPLIT && DP <= 64;
+    static constexpr int BYTES = (TWICE ? 2 : 1) * ONE;
+};
+
+template <typename T, int DP> __device__ __forceinline__ bool fwd_pass(const Args& a, unsigned char* smem) {
     using LY = Lay<T, DP>;
-    __shared__ __align__(16) unsigned char smem[LY::NATB + (LY::NATSEQ ? LY::NATB : LY::TRB)];
-    T* Kn = reinterpret_cast<T*>(smem);
-    T* Vt = reinterpret_cast<T*>(smem + LY::NATB);
+    using FS = FwdSmem<T, DP>;
     const WaveIds w = wave_ids();
     const int W = w.nthr >> 6;
     int bh, blk;
@@ -119,8 +148,6 @@ template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512)
     const int own = row0 + w.l16;
     const bool active = row0 < L;
     const Src<T, 2> src = {{slice<T>(a.k, b, h), slice<T>(a.v, b, h)}, {a.k.sl, a.v.sl}};
-    T* const nat[2] = {Kn, nullptr};
-    T* const tr[2] = {nullptr, Vt};
     Stage<T, DP, 2> stg;
     stg.load(src, 0, L, D, w.tid, w.nthr);
 
@@ -132,12 +159,16 @@ template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512)
     for (int t = 0; t < LY::NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float sc = a.scale;
 
-    for (int x0 = 0; x0 < L; x0 += CH) {
-        lds_barrier();
+    const auto store = [&](int buf) {
+        T* const Kn = reinterpret_cast<T*>(smem + buf * FS::ONE);
+        T* const nat[2] = {Kn, nullptr};
+        T* const tr[2] = {nullptr, reinterpret_cast<T*>(smem + buf * FS::ONE + LY::NATB)};
         stg.store(nat, tr, w.tid, w.nthr);
-        lds_barrier();
-        if (x0 + CH < L) stg.load(src, x0 + CH, L, D, w.tid, w.nthr);
-        if (!active) continue;
+    };
+    const auto compute = [&](int x0, int buf) {
+        if (!active) return;
+        const T* Kn = reinterpret_cast<const T*>(smem + buf * FS::ONE);
+        const T* Vt = reinterpret_cast<const T*>(smem + buf * FS::ONE + LY::NATB);
         f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
         mma_d<T, DP>(s0, Kn, qf, w.l16, w.g);
         mma_d<T, DP>(s1, Kn + 16 * LY::PN, qf, w.l16, w.g);
@@ -166,14 +197,42 @@ template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512)
             acc[t] = mma_seq<T>(acc[t] * alpha, va, pb);
         }
         m = mnew;
+    };
+    if constexpr (FS::TWICE) {
+        lds_barrier();  // nobody reads the buffers any more (a redone pass)
+        store(0);
+        if (CH < L) stg.load(src, CH, L, D, w.tid, w.nthr);
+        for (int x0 = 0, buf = 0; x0 < L; x0 += CH, buf ^= 1) {
+            lds_barrier();  // chunk x0 written; the other buffer's chunk read by everyone
+            if (x0 + CH < L) store(buf ^ 1);
+            if (x0 + 2 * CH < L) stg.load(src, x0 + 2 * CH, L, D, w.tid, w.nthr);
+            compute(x0, buf);
+        }
+    } else {
+        for (int x0 = 0; x0 < L; x0 += CH) {
+            lds_barrier();
+            store(0);
+            lds_barrier();
+            if constexpr (ET<T>::SPLIT) compute(x0, 0);
+            if (x0 + CH < L) stg.load(src, x0 + CH, L, D, w.tid, w.nthr);
+            if constexpr (!ET<T>::SPLIT) compute(x0, 0);
+        }
     }
-    if (!active) return;
+    if (!active) return false;
     lsum = xsum4(lsum);
+    const float nan = total(acc) + lsum;
     if (own < L) {
         const int64_t r = (int64_t)bh * L + own;
         store_rows<T, DP>(a.out0, r * D, acc, 1.f / lsum, D, w.g);
         if (w.g == 0) a.lse_out[r] = m + logf(lsum);
     }
+    return own < L && nan != nan;
+}
+
+// Wider rows than DP = 128 run 256-thread workgroups (one wave per SIMD, every register for the wave).
+template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512) void k_fwd(Args a) {
+    __shared__ __align__(16) unsigned char smem[FwdSmem<T, DP>::BYTES];
+    redo_if_nan<T>([&](auto t) { return fwd_pass<decltype(t), DP>(a, smem); });
 }
 
 // =====================================================================================================================
@@ -259,6 +318,10 @@ template <typename T, int DP, bool FUSED> struct BwdRow {
 #pragma unroll
         for (int t = 0; t < LY::NT; ++t) acc[t] = mma_seq<T>(acc[t], read_seqa<T, DP>(Kt, t, w.l16, w.g), dsb);
     }
+    __device__ __forceinline__ bool nan(int L) const {
+        const float v = total(acc);
+        return active && own < L && v != v;
+    }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) store_rows<T, DP>(a.out0, ((int64_t)bh * a.L + own) * a.D, acc, a.scale, a.D, w.g);
     }
@@ -325,6 +388,10 @@ template <typename T, int DP> struct BwdCol {
             av[t] = mma_seq<T>(av[t], read_seqa<T, DP>(Ot, t, w.l16, w.g), pb);
             ak[t] = mma_seq<T>(ak[t], read_seqa<T, DP>(Qt, t, w.l16, w.g), dsb);
         }
+    }
+    __device__ __forceinline__ bool nan(int L) const {
+        const float v = total(ak) + total(av);
+        return active && own < L && v != v;
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) {
@@ -423,20 +490,48 @@ template <typename T, int DP, bool FUSED> struct BbRow {
                 t_acc += m1[hh][r];
             }
         }
-        const SeqB<T> pb = make_seqb<T>(p[0], p[1]);
-        const SeqB<T> dsb = make_seqb<T>(ds[0], ds[1]);
-        const SeqB<T> pab = make_seqb<T>(pa[0], pa[1]);
-        const SeqB<T> m1b = make_seqb<T>(m1[0], m1[1]);
+        if constexpr (ET<T>::SPLIT) {
+            // One operand's planes at a time (twelve registers each): all four beside the accumulators and the own
+            // rows' planes would leave a SIMD one wave. K^T is read three times for it.
+            auto add = [&](f32x4(&acc)[LY::NT], const T* Xt, const SeqB<T>& o) {
 #pragma unroll
-        for (int t = 0; t < LY::NT; ++t) {
-            const SeqA<T> ka = read_seqa<T, DP>(Kt, t, w.l16, w.g);
-            X[t] = mma_seq<T>(X[t], ka, m1b);
-            U[t] = mma_seq<T>(U[t], ka, dsb);
-            Z[t] = mma_seq<T>(Z[t], ka, pb);
-            X[t] = mma_seq<T>(X[t], read_seqa<T, DP>(gKt, t, w.l16, w.g), dsb);
-            Wv[t] = mma_seq<T>(Wv[t], read_seqa<T, DP>(Vt, t, w.l16, w.g), pab);
-            Wv[t] = mma_seq<T>(Wv[t], read_seqa<T, DP>(gVt, t, w.l16, w.g), pb);
+                for (int t = 0; t < LY::NT; ++t) acc[t] = mma_seq<T>(acc[t], read_seqa<T, DP>(Xt, t, w.l16, w.g), o);
+            };
+            {
+                const SeqB<T> o = make_seqb<T>(m1[0], m1[1]);
+                add(X, Kt, o);
+            }
+            {
+                const SeqB<T> o = make_seqb<T>(ds[0], ds[1]);
+                add(U, Kt, o);
+                add(X, gKt, o);
+            }
+            {
+                const SeqB<T> o = make_seqb<T>(p[0], p[1]);
+                add(Z, Kt, o);
+                add(Wv, gVt, o);
+            }
+            add(Wv, Vt, make_seqb<T>(pa[0], pa[1]));
+        } else {
+            const SeqB<T> pb = make_seqb<T>(p[0], p[1]);
+            const SeqB<T> dsb = make_seqb<T>(ds[0], ds[1]);
+            const SeqB<T> pab = make_seqb<T>(pa[0], pa[1]);
+            const SeqB<T> m1b = make_seqb<T>(m1[0], m1[1]);
+#pragma unroll
+            for (int t = 0; t < LY::NT; ++t) {
+                const SeqA<T> ka = read_seqa<T, DP>(Kt, t, w.l16, w.g);
+                X[t] = mma_seq<T>(X[t], ka, m1b);
+                U[t] = mma_seq<T>(U[t], ka, dsb);
+                Z[t] = mma_seq<T>(Z[t], ka, pb);
+                X[t] = mma_seq<T>(X[t], read_seqa<T, DP>(gKt, t, w.l16, w.g), dsb);
+                Wv[t] = mma_seq<T>(Wv[t], read_seqa<T, DP>(Vt, t, w.l16, w.g), pab);
+                Wv[t] = mma_seq<T>(Wv[t], read_seqa<T, DP>(gVt, t, w.l16, w.g), pb);
+            }
         }
+    }
+    __device__ __forceinline__ bool nan(int L) const {
+        const float v = total(X) + total(U) + total(Z) + total(Wv) + e_acc + t_acc;
+        return active && own < L && v != v;
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w, float* st) {
         const float E = xsum4(e_acc);
@@ -556,6 +651,10 @@ template <typename T, int DP> struct BbCol {
             hv[t] = mma_seq<T>(hv[t], read_seqa<T, DP>(Ot, t, w.l16, w.g), pab);
         }
     }
+    __device__ __forceinline__ bool nan(int L) const {
+        const float v = total(hk) + total(hv);
+        return active && own < L && v != v;
+    }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) {
             const int64_t r = ((int64_t)bh * a.L + own) * a.D;
@@ -574,7 +673,8 @@ template <typename T, int DP> struct BbCol {
 template <int NS> struct NoStats {};
 
 template <typename T, int DP, class Row, class Col, int NCOL, int NSTAT>
-__device__ __forceinline__ void fused_two_pass(const Args& a, unsigned char* smem, float* st) {
+__device__ __forceinline__ bool fused_two_pass(const Args& a, unsigned char* smem, float* st) {
+    constexpr bool LATE = loads_after<T>();
     const WaveIds w = wave_ids();
     const int bh = blockIdx.x;
     const int b = bh / a.H, h = bh - b * a.H;
@@ -609,12 +709,14 @@ __device__ __forceinline__ void fused_two_pass(const Args& a, unsigned char* sme
         lds_barrier();
         rst.store(rn, rt, w.tid, w.nthr);
         lds_barrier();
+        if constexpr (LATE) row.chunk(a, x0, smem, w);
         if (x0 + CH < L)
             rst.load(rsrc, x0 + CH, L, D, w.tid, w.nthr);
         else
             cst.load(csrc, 0, L, D, w.tid, w.nthr);
-        row.chunk(a, x0, smem, w);
+        if constexpr (!LATE) row.chunk(a, x0, smem, w);
     }
+    bool nan = row.nan(L);
     if constexpr (NSTAT == 1) {
         row.finish(a, w);
     } else {
@@ -625,10 +727,12 @@ __device__ __forceinline__ void fused_two_pass(const Args& a, unsigned char* sme
         lds_barrier();
         cst.store(cn, ct, w.tid, w.nthr);
         lds_barrier();
+        if constexpr (LATE) col.chunk(a, smem, st + x0, STAT_MAX, w);
         if (x0 + CH < L) cst.load(csrc, x0 + CH, L, D, w.tid, w.nthr);
-        col.chunk(a, smem, st + x0, STAT_MAX, w);
+        if constexpr (!LATE) col.chunk(a, smem, st + x0, STAT_MAX, w);
     }
     col.finish(a, w);
+    return nan || col.nan(L);
 }
 
 template <typename T, int DP> struct FusedSmem {
@@ -641,13 +745,19 @@ template <typename T, int DP> struct FusedSmem {
 template <typename T, int DP> __global__ __launch_bounds__(512) void k_bwd_fused(Args a) {
     __shared__ __align__(16) unsigned char smem[FusedSmem<T, DP>::BWD];
     __shared__ __align__(16) float st[2 * STAT_MAX];
-    fused_two_pass<T, DP, BwdRow<T, DP, true>, BwdCol<T, DP>, 2, 1>(a, smem, st);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return fused_two_pass<U, DP, BwdRow<U, DP, true>, BwdCol<U, DP>, 2, 1>(a, smem, st);
+    });
 }
 
 template <typename T, int DP> __global__ __launch_bounds__(512) void k_bb_fused(Args a) {
     __shared__ __align__(16) unsigned char smem[FusedSmem<T, DP>::BB];
     __shared__ __align__(16) float st[4 * STAT_MAX];
-    fused_two_pass<T, DP, BbRow<T, DP, true>, BbCol<T, DP>, 3, 3>(a, smem, st);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return fused_two_pass<U, DP, BbRow<U, DP, true>, BbCol<U, DP>, 3, 3>(a, smem, st);
+    });
 }
 
 #include "attn_resident.hpp"
@@ -655,7 +765,8 @@ template <typename T, int DP> __global__ __launch_bounds__(512) void k_bb_fused(
 
 // Two-launch row kernel: own rows [blk * 16 W, (blk + 1) * 16 W) of one (b, h); statistics go to a.stats.
 template <typename T, int DP, class Row, int NROW, bool BB>
-__device__ __forceinline__ void stream_row(const Args& a, unsigned char* smem) {
+__device__ __forceinline__ bool stream_row(const Args& a, unsigned char* smem) {
+    constexpr bool LATE = loads_after<T>();
     const WaveIds w = wave_ids();
     int bh, blk;
     decode_block(a, bh, blk);
@@ -677,19 +788,23 @@ __device__ __forceinline__ void stream_row(const Args& a, unsigned char* smem) {
         lds_barrier();
         rst.store(rn, rt, w.tid, w.nthr);
         lds_barrier();
+        if constexpr (LATE) row.chunk(a, x0, smem, w);
         if (x0 + CH < L) rst.load(src, x0 + CH, L, D, w.tid, w.nthr);
-        row.chunk(a, x0, smem, w);
+        if constexpr (!LATE) row.chunk(a, x0, smem, w);
     }
+    const bool nan = row.nan(L);
     if constexpr (BB) {
         row.finish(a, w, nullptr);
     } else {
         row.finish(a, w);
     }
+    return nan;
 }
 
 // Two-launch col kernel: own rows [blk * 16 W, (blk + 1) * 16 W) of one (b, h); statistics staged from a.lse/a.stats.
 template <typename T, int DP, class Col, int NCOL, int NSTAT>
-__device__ __forceinline__ void stream_col(const Args& a, unsigned char* smem) {
+__device__ __forceinline__ bool stream_col(const Args& a, unsigned char* smem) {
+    constexpr bool LATE = loads_after<T>();
     const WaveIds w = wave_ids();
     int bh, blk;
     decode_block(a, bh, blk);
@@ -700,10 +815,10 @@ __device__ __forceinline__ void stream_col(const Args& a, unsigned char* smem) {
     T* cn[NCOL];
     T* ct[NCOL];
     col.lds(smem, cn, ct);
-    float* stc = reinterpret_cast<float*>(smem + Col::SMEM);
     Stage<T, DP, NCOL> cst;
     StatStage<NSTAT> sst;
     const int64_t rb = (int64_t)bh * L;
+    float* stc = reinterpret_cast<float*>(smem + Col::SMEM);
     cst.load(src, 0, L, D, w.tid, w.nthr);
     sst.load(a.lse, a.stats, a.bhl, rb, 0, L, w.tid);
     col.init(a, bh, blk * (w.nthr >> 2), w);
@@ -712,33 +827,51 @@ __device__ __forceinline__ void stream_col(const Args& a, unsigned char* smem) {
         cst.store(cn, ct, w.tid, w.nthr);
         sst.store(stc, w.tid);
         lds_barrier();
+        if constexpr (LATE) col.chunk(a, smem, stc, CH, w);
         if (x0 + CH < L) {
             cst.load(src, x0 + CH, L, D, w.tid, w.nthr);
             sst.load(a.lse, a.stats, a.bhl, rb, x0 + CH, L, w.tid);
         }
-        col.chunk(a, smem, stc, CH, w);
+        if constexpr (!LATE) col.chunk(a, smem, stc, CH, w);
     }
     col.finish(a, w);
+    return col.nan(L);
 }
 
 template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_row(Args a) {
     __shared__ __align__(16) unsigned char smem[BwdRow<T, DP, false>::SMEM];
-    stream_row<T, DP, BwdRow<T, DP, false>, 2, false>(a, smem);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return stream_row<U, DP, BwdRow<U, DP, false>, 2, false>(a, smem);
+    });
 }
 
 template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_col(Args a) {
     __shared__ __align__(16) unsigned char smem[BwdCol<T, DP>::SMEM + 2 * CH * 4];
-    stream_col<T, DP, BwdCol<T, DP>, 2, 1>(a, smem);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return stream_col<U, DP, BwdCol<U, DP>, 2, 1>(a, smem);
+    });
 }
 
-template <typename T, int DP> __global__ __launch_bounds__(256) void k_bb_row(Args a) {
+// The split backward-of-backward kernels at two waves per SIMD (256 registers): left alone, the compiler took 280 to
+// 340 at D = 64, one workgroup per CU.
+#define BB_SPLIT_WAVES(T, DP) __attribute__((amdgpu_waves_per_eu(ET<T>::SPLIT && DP <= 64 ? 2 : 1, 8)))
+
+template <typename T, int DP> __global__ __launch_bounds__(256) BB_SPLIT_WAVES(T, DP) void k_bb_row(Args a) {
     __shared__ __align__(16) unsigned char smem[BbRow<T, DP, false>::SMEM];
-    stream_row<T, DP, BbRow<T, DP, false>, 4, true>(a, smem);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return stream_row<U, DP, BbRow<U, DP, false>, 4, true>(a, smem);
+    });
 }
 
-template <typename T, int DP> __global__ __launch_bounds__(256) void k_bb_col(Args a) {
+template <typename T, int DP> __global__ __launch_bounds__(256) BB_SPLIT_WAVES(T, DP) void k_bb_col(Args a) {
     __shared__ __align__(16) unsigned char smem[BbCol<T, DP>::SMEM + 4 * CH * 4];
-    stream_col<T, DP, BbCol<T, DP>, 3, 3>(a, smem);
+    redo_if_nan<T>([&](auto t) {
+        using U = decltype(t);
+        return stream_col<U, DP, BbCol<U, DP>, 3, 3>(a, smem);
+    });
 }
 
 // =====================================================================================================================
@@ -846,25 +979,41 @@ static int persistent_grid(const void* kernel, int threads, int64_t work) {
 
 #include "attn_f64.hpp"
 
-template <template <typename, int> class F, typename... Rest>
-static int dispatch(int dtype, int D, Rest&&... rest) {
+// fp32 widths whose one-workgroup kernels (L <= 128) run as split products.
+template <typename T> constexpr bool one_workgroup(int dp) { return dp <= (ET<T>::SPLIT ? 32 : 128); }
+
+// fp32 as split products (f32s): every L > 128, and D in 17..32 from L = 33 on. Against the fp32 MFMA, forward /
+// backward / bwd_bwd in us: 64 slices, L = 400, D = 64: 31.6 / 85 / 185 against 41 / 126 / 328; 8 slices, L = 300,
+// D = 128: 28 / 89 / 196 against 38 / 116 / 287; 512 slices, L = 100, D = 32: 13 / 31 / 69 against 16 / 40 / 102. Below
+// those lines it loses: a wave that runs both passes of bwd_bwd spills from D = 64 on (50 against 37 at 256 slices,
+// L = 64, D = 64; 474 against 309 at 128 slices, L = 100, D = 128), and one chunk is mostly its own split and stores
+// (2,048 slices, L = 30, D = 128: 42 / 141 / 716 against 29 / 112 / 618). The three ops of a shape take the same side,
+// so that P is recomputed with the scores' own rounding.
+static bool split_f32(int L, int D) { return D > 16 && D <= 128 && (L > STAT_MAX || (D <= 32 && L > CH)); }
+
+template <template <typename, int> class F> static int dispatch(int dtype, int D, const Args& rest, hipStream_t s) {
     if (dtype == EBR_DTYPE_F32) {
-        if (D <= 16) return F<float, 16>::run(rest...);
-        if (D <= 32) return F<float, 32>::run(rest...);
-        if (D <= 64) return F<float, 64>::run(rest...);
-        if (D <= 128) return F<float, 128>::run(rest...);
-        return F<float, DMAX_WIDE>::run(rest...);
+        if (split_f32(rest.L, D)) {
+            if (D <= 32) return F<f32s, 32>::run(rest, s);
+            if (D <= 64) return F<f32s, 64>::run(rest, s);
+            return F<f32s, 128>::run(rest, s);
+        }
+        if (D <= 16) return F<float, 16>::run(rest, s);
+        if (D <= 32) return F<float, 32>::run(rest, s);
+        if (D <= 64) return F<float, 64>::run(rest, s);
+        if (D <= 128) return F<float, 128>::run(rest, s);
+        return F<float, DMAX_WIDE>::run(rest, s);
     }
     if (dtype == EBR_DTYPE_BF16) {
-        if (D <= 32) return F<__bf16, 32>::run(rest...);
-        if (D <= 64) return F<__bf16, 64>::run(rest...);
-        if (D <= 128) return F<__bf16, 128>::run(rest...);
-        return F<__bf16, DMAX_WIDE>::run(rest...);
+        if (D <= 32) return F<__bf16, 32>::run(rest, s);
+        if (D <= 64) return F<__bf16, 64>::run(rest, s);
+        if (D <= 128) return F<__bf16, 128>::run(rest, s);
+        return F<__bf16, DMAX_WIDE>::run(rest, s);
     }
-    if (D <= 32) return F<_Float16, 32>::run(rest...);
-    if (D <= 64) return F<_Float16, 64>::run(rest...);
-    if (D <= 128) return F<_Float16, 128>::run(rest...);
-    return F<_Float16, DMAX_WIDE>::run(rest...);
+    if (D <= 32) return F<_Float16, 32>::run(rest, s);
+    if (D <= 64) return F<_Float16, 64>::run(rest, s);
+    if (D <= 128) return F<_Float16, 128>::run(rest, s);
+    return F<_Float16, DMAX_WIDE>::run(rest, s);
 }
 
 // The long-sequence kernels (16-bit inputs, L > 128): D a full chunk width, 32-bit buffer offsets per slice.
@@ -917,7 +1066,7 @@ static bool plan_allows(const Args& a, int f) { return a.plan == EBR_PLAN_AUTO |
 template <typename T, int DP> struct FwdLaunch {
     static int run(Args a, hipStream_t s) {
         const int64_t bh = (int64_t)a.B * a.H;
-        if constexpr (!ET<T>::F32 && DP <= 128) {
+        if constexpr (!ET<T>::WIDE && DP <= 128) {
             if (plan_allows(a, EBR_PLAN_RESIDENT) && resident_shape(a, DP, 2, false)) {
                 a.nblk = 1;
                 const dim3 grid((int)bh), block(fused_threads(a.L));
@@ -930,7 +1079,7 @@ template <typename T, int DP> struct FwdLaunch {
                 return launch_rc();
             }
         }
-        if constexpr (!ET<T>::F32 && DP <= 128) {
+        if constexpr (!ET<T>::WIDE && DP <= 128) {
             if (plan_allows(a, EBR_PLAN_LONG) && long_shape(a, DP, false)) {  // streamed stages, a loader wave
                 auto run = [&](auto nw) {
                     constexpr int NW = decltype(nw)::value;
@@ -961,7 +1110,7 @@ template <typename T, int DP> struct FwdLaunch {
 template <typename T, int DP> struct BwdLaunch {
     static int run(Args a, hipStream_t s) {
         const int64_t bh = (int64_t)a.B * a.H;
-        if constexpr (!ET<T>::F32 && DP <= 128) {
+        if constexpr (!ET<T>::WIDE && DP <= 128) {
             a.gq = a.gk = a.gv = a.dO;  // only q, k, v, dO are read
             if ((plan_allows(a, EBR_PLAN_PERSISTENT) || a.plan == EBR_PLAN_RESIDENT) &&
                 resident_shape(a, DP, 2, true)) {
@@ -1022,7 +1171,7 @@ template <typename T, int DP> struct BwdLaunch {
                 return launch_rc();
             }
         }
-        if constexpr (!ET<T>::F32 && DP <= 128) {
+        if constexpr (!ET<T>::WIDE && DP <= 128) {
             if (plan_allows(a, EBR_PLAN_LONG) && long_shape(a, DP, true)) {  // k_bwd_long_row, k_bwd_long_col
                 auto run = [&](auto nw) {
                     constexpr int NW = decltype(nw)::value;
@@ -1041,7 +1190,8 @@ template <typename T, int DP> struct BwdLaunch {
             }
         }
         if (!plan_allows(a, EBR_PLAN_GENERIC)) return EBR_ERR_PLAN;
-        if constexpr (DP <= 128) {  // wider rows take the two launches at any L (512-thread workgroups would spill)
+        // wider rows take the two launches at any L (512-thread workgroups would spill)
+        if constexpr (one_workgroup<T>(DP)) {
             if (fused_shape(a.L)) {
                 a.nblk = 1;
                 a.xcd_remap = 0;
@@ -1080,8 +1230,8 @@ template <typename T, int DP> struct BbLaunch {
             if (a.plan == EBR_PLAN_LONG) return EBR_ERR_PLAN;
             if (a.plan == EBR_PLAN_GENERIC || !resident_shape(a, DP, (int)sizeof(T), true)) {
                 if (!plan_allows(a, EBR_PLAN_GENERIC)) return EBR_ERR_PLAN;
-                hipLaunchKernelGGL((k_bb_fused<T, DP>), grid, block, 0, s, a);
-            } else if constexpr (!ET<T>::F32) {
+                if constexpr (one_workgroup<T>(DP)) hipLaunchKernelGGL((k_bb_fused<T, DP>), grid, block, 0, s, a);
+            } else if constexpr (!ET<T>::WIDE) {
                 const int nch = (a.L + CH - 1) / CH;
                 // tiles shared through LDS, persistent with loader waves (k_bb_share), where its regions fit the LDS:
                 // D <= 64 up to three chunks, D = 128 up to two
@@ -1117,7 +1267,7 @@ template <typename T, int DP> struct BbLaunch {
             }
             return launch_rc();
         }
-        if constexpr (!ET<T>::F32 && DP <= 128) {
+        if constexpr (!ET<T>::WIDE && DP <= 128) {
             if (plan_allows(a, EBR_PLAN_LONG) && long_shape(a, DP, true)) {  // k_bb_long_row, k_bb_long_col
                 auto run = [&](auto nw) {
                     constexpr int NW = decltype(nw)::value;
