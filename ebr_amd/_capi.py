@@ -111,9 +111,15 @@ SIGNATURES = {
     # include/ebr_block.h
     "ebr_block_rmsnorm": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_float] + [_P] * 3),
     "ebr_block_rmsnorm_bwd": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_float] + [_P] * 4),
+    "ebr_block_rmsnorm_bwd_add": (
+        ctypes.c_int,
+        [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_float] + [_P] * 5,
+    ),
+    "ebr_block_add_rmsnorm": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_float] + [_P] * 5),
     "ebr_block_rmsnorm_bwd2": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_float] + [_P] * 6),
     "ebr_block_swiglu": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 3),
     "ebr_block_swiglu_bwd": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 4),
+    "ebr_block_swiglu_bwd_add": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 5),
     "ebr_block_swiglu_bwd2": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 6),
     "ebr_attn_error_string": (ctypes.c_char_p, [ctypes.c_int]),
     "ebr_attn_abi_version": (ctypes.c_int, []),

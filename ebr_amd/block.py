@@ -273,6 +273,13 @@ def rms_norm(x: Tensor, eps: float) -> Tensor:
     return _RmsNorm.apply(x, eps)
 
 
+def add_rms_norm(x: Tensor, r: Tensor, eps: float) -> Tensor:
+    """``rms_norm(x + r, eps)``: the residual sum rounded to the dtype, then its norm, in one kernel on the native path."""
+    host = None if torch.compiler.is_compiling() else _host.module()
+    y = None if host is None else host.add_rms_norm(x, r, eps)
+    return rms_norm(x + r, eps) if y is None else y
+
+
 def swiglu(gate_up: Tensor) -> Tensor:
     """silu(gate) * up of the two halves of the last dim, differentiable twice."""
     host = _host.module()
@@ -286,4 +293,4 @@ def swiglu(gate_up: Tensor) -> Tensor:
 rms_norm = torch._dynamo.allow_in_graph(rms_norm)
 swiglu = torch._dynamo.allow_in_graph(swiglu)
 
-__all__ = ["rms_norm", "swiglu"]
+__all__ = ["add_rms_norm", "rms_norm", "swiglu"]

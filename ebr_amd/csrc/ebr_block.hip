@@ -13,6 +13,13 @@
 //   backward2 (cotangents cg, cu of dg, du): gg = cg dy u silu''(g) + cu dy silu'(g), gu = cg dy silu'(g),
 //   gdy = cg u silu'(g) + cu silu(g); with s = sigmoid(g): silu' = s (1 + g (1 - s)),
 //   silu'' = s (1 - s) (2 + g (1 - 2 s)).
+//
+// Sums with a tensor that would otherwise be kernels of their own are taken where the operand is in registers anyway,
+// with the same two roundings: the residual sum before a norm (mode 4) and the sum of a backward with a gradient that
+// is already there (mode 3), as the second derivative of a block adds up twice per norm and once per SwiGLU. A separate
+// sum reads two tensors and writes one; folded in, it costs one read (and the residual sum's write). Measured in bf16,
+// kernel and sum apart -> together: residual sum and norm at [31104, 512] 28.6 -> 24.5 us (5.2 TB/s; 51 -> 42 at
+// [64000, 512], 6.2 TB/s), norm backward 34 -> 21, SwiGLU backward at [31104, 2 x 1536] 181 -> 128 (6.0 TB/s).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -56,14 +63,22 @@ template <typename T> __device__ __forceinline__ void stv(T* p, const Vec<T>& v)
 constexpr int WAVES_PER_BLOCK = 4;
 
 struct NormArgs {
-    const void *x, *dy, *c;
-    void *y, *gx, *gdy;
+    const void *x, *dy, *c;  // mode 3: c is the gradient to add; mode 4: dy is the second summand
+    void *y, *gx, *gdy;      // mode 4: gx is the sum
     int64_t rows;
     int C;
     float eps;
 };
 
-// Per-row factors of the three rms_norm modes, from the row sums (already reduced over the wave).
+// round(v + a) of a value already rounded to T, kept opaque so that both roundings happen.
+template <typename T, typename A> __device__ __forceinline__ T add_rounded(T v, A a) {
+#pragma clang fp contract(off)
+    A w = wide<T, A>(v);
+    asm volatile("" : "+v"(w));
+    return narrow<T, A>(w + a);
+}
+
+// Per-row factors of the rms_norm modes, from the row sums (already reduced over the wave).
 template <typename A> struct NormRow {
     A r, r3c, sdx, scx, kx;
 };
@@ -79,12 +94,17 @@ template <typename A, int MODE> __device__ __forceinline__ NormRow<A> norm_row(A
     return f;
 }
 
-// mode 0: o0 = y; 1: o0 = dx; 2: o0 = gx, o1 = gdy.
+// mode 0: o0 = y; 1: o0 = dx; 2: o0 = gx, o1 = gdy; 3: o0 = round(dx) + c; 4: o0 = y of the sum xv, o1 = the sum.
 template <typename T, typename A, int MODE>
 __device__ __forceinline__ void norm_out(const NormRow<A>& f, A xv, A dv, A cv, T& o0, T& o1) {
 #pragma clang fp contract(off)
     if constexpr (MODE == 0) o0 = narrow<T, A>(xv * f.r);
     if constexpr (MODE == 1) o0 = narrow<T, A>(f.r * dv - f.r3c * f.sdx * xv);
+    if constexpr (MODE == 3) o0 = add_rounded<T, A>(narrow<T, A>(f.r * dv - f.r3c * f.sdx * xv), cv);
+    if constexpr (MODE == 4) {
+        o0 = narrow<T, A>(xv * f.r);
+        o1 = narrow<T, A>(xv);
+    }
     if constexpr (MODE == 2) {
         o0 = narrow<T, A>(f.kx * xv - f.r3c * f.sdx * cv - f.r3c * f.scx * dv);
         o1 = narrow<T, A>(f.r * cv - f.r3c * f.scx * xv);
@@ -101,29 +121,33 @@ template <typename T, int MODE> __global__ __launch_bounds__(64 * WAVES_PER_BLOC
     const int C = a.C;
     const T* x = reinterpret_cast<const T*>(a.x) + row * C;
     const T* dy = MODE >= 1 ? reinterpret_cast<const T*>(a.dy) + row * C : nullptr;
-    const T* c = MODE == 2 ? reinterpret_cast<const T*>(a.c) + row * C : nullptr;
+    const T* c = MODE == 2 || MODE == 3 ? reinterpret_cast<const T*>(a.c) + row * C : nullptr;
+    const auto in = [&](int k) {  // the row's element, mode 4: of the sum
+        if constexpr (MODE == 4) return wide<T, A>(add_rounded<T, A>(x[k], wide<T, A>(dy[k])));
+        return wide<T, A>(x[k]);
+    };
     A sxx = 0, sdx = 0, scx = 0, scd = 0;
     for (int k = lane; k < C; k += 64) {
-        const A xv = wide<T, A>(x[k]);
+        const A xv = in(k);
         sxx += xv * xv;
-        if constexpr (MODE >= 1) sdx += wide<T, A>(dy[k]) * xv;
+        if constexpr (MODE >= 1 && MODE < 4) sdx += wide<T, A>(dy[k]) * xv;
         if constexpr (MODE == 2) {
             const A cv = wide<T, A>(c[k]);
             scx += cv * xv;
             scd += cv * wide<T, A>(dy[k]);
         }
     }
-    const NormRow<A> f = norm_row<A, MODE>(wave_sum(sxx), MODE >= 1 ? wave_sum(sdx) : (A)0,
+    const NormRow<A> f = norm_row<A, MODE>(wave_sum(sxx), MODE >= 1 && MODE < 4 ? wave_sum(sdx) : (A)0,
                                            MODE == 2 ? wave_sum(scx) : (A)0, MODE == 2 ? wave_sum(scd) : (A)0, C,
                                            a.eps);
     T* o0 = reinterpret_cast<T*>(MODE == 2 ? a.gx : a.y) + row * C;
-    T* o1 = MODE == 2 ? reinterpret_cast<T*>(a.gdy) + row * C : nullptr;
+    T* o1 = MODE == 2 || MODE == 4 ? reinterpret_cast<T*>(MODE == 2 ? a.gdy : a.gx) + row * C : nullptr;
     for (int k = lane; k < C; k += 64) {
         T r0, r1;
-        norm_out<T, A, MODE>(f, wide<T, A>(x[k]), MODE >= 1 ? wide<T, A>(dy[k]) : (A)0,
-                             MODE == 2 ? wide<T, A>(c[k]) : (A)0, r0, r1);
+        norm_out<T, A, MODE>(f, in(k), MODE >= 1 && MODE < 4 ? wide<T, A>(dy[k]) : (A)0,
+                             MODE == 2 || MODE == 3 ? wide<T, A>(c[k]) : (A)0, r0, r1);
         o0[k] = r0;
-        if constexpr (MODE == 2) o1[k] = r1;
+        if constexpr (MODE == 2 || MODE == 4) o1[k] = r1;
     }
 }
 
@@ -153,8 +177,17 @@ __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void k_rmsnorm_vec(NormArgs a
             const int64_t off = row * C + (k < C ? k : 0);
             xv[r][v] = ldv(X + off);
             if constexpr (MODE >= 1) dv[r][v] = ldv(DY + off);
-            if constexpr (MODE == 2) cv[r][v] = ldv(CC + off);
+            if constexpr (MODE == 2 || MODE == 3) cv[r][v] = ldv(CC + off);
         }
+    }
+    if constexpr (MODE == 4) {
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e)
+                    xv[r][v].e[e] = add_rounded<T, A>(xv[r][v].e[e], wide<T, A>(dv[r][v].e[e]));
     }
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
@@ -166,7 +199,7 @@ __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void k_rmsnorm_vec(NormArgs a
             for (int e = 0; e < VEC; ++e) {
                 const A xe = wide<T, A>(xv[r][v].e[e]);
                 sxx += xe * xe;
-                if constexpr (MODE >= 1) sdx += wide<T, A>(dv[r][v].e[e]) * xe;
+                if constexpr (MODE >= 1 && MODE < 4) sdx += wide<T, A>(dv[r][v].e[e]) * xe;
                 if constexpr (MODE == 2) {
                     const A ce = wide<T, A>(cv[r][v].e[e]);
                     scx += ce * xe;
@@ -174,13 +207,13 @@ __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void k_rmsnorm_vec(NormArgs a
                 }
             }
         }
-        const NormRow<A> f = norm_row<A, MODE>(wave_sum(sxx), MODE >= 1 ? wave_sum(sdx) : (A)0,
+        const NormRow<A> f = norm_row<A, MODE>(wave_sum(sxx), MODE >= 1 && MODE < 4 ? wave_sum(sdx) : (A)0,
                                                MODE == 2 ? wave_sum(scx) : (A)0, MODE == 2 ? wave_sum(scd) : (A)0, C,
                                                a.eps);
         if (row0 + r >= a.rows) break;  // wave-uniform
         const int64_t base = (row0 + r) * C;
         T* O0 = reinterpret_cast<T*>(MODE == 2 ? a.gx : a.y) + base;
-        T* O1 = MODE == 2 ? reinterpret_cast<T*>(a.gdy) + base : nullptr;
+        T* O1 = MODE == 2 || MODE == 4 ? reinterpret_cast<T*>(MODE == 2 ? a.gdy : a.gx) + base : nullptr;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int k = (v * 64 + lane) * VEC;
@@ -188,16 +221,17 @@ __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void k_rmsnorm_vec(NormArgs a
             Vec<T> r0, r1;
 #pragma unroll
             for (int e = 0; e < VEC; ++e)
-                norm_out<T, A, MODE>(f, wide<T, A>(xv[r][v].e[e]), MODE >= 1 ? wide<T, A>(dv[r][v].e[e]) : (A)0,
-                                     MODE == 2 ? wide<T, A>(cv[r][v].e[e]) : (A)0, r0.e[e], r1.e[e]);
+                norm_out<T, A, MODE>(f, wide<T, A>(xv[r][v].e[e]),
+                                     MODE >= 1 && MODE < 4 ? wide<T, A>(dv[r][v].e[e]) : (A)0,
+                                     MODE == 2 || MODE == 3 ? wide<T, A>(cv[r][v].e[e]) : (A)0, r0.e[e], r1.e[e]);
             stv(O0 + k, r0);
-            if constexpr (MODE == 2) stv(O1 + k, r1);
+            if constexpr (MODE == 2 || MODE == 4) stv(O1 + k, r1);
         }
     }
 }
 
 struct GluArgs {
-    const void *gu, *dy, *c;
+    const void *gu, *dy, *c;  // mode 3: c is the gradient to add
     void *y, *ggu, *gdy;
     int64_t n;  // rows
     int I;      // half width
@@ -207,7 +241,8 @@ template <typename A> __device__ __forceinline__ A sigmoid_of(A g) { return (A)1
 
 // One element of SwiGLU. mode 0: o0 = y = silu(g) u; 1: o0 = dg, o1 = du given dy; 2: o0 = gg, o1 = gu, o2 = gdy
 // given dy and the cotangents (cg, cu) of (dg, du). The 16-bit roundings of modes 0 and 1 are where eager autograd
-// rounds: silu is rounded before the product; dg = round(round(dy u) silu'), du = round(dy round(silu)).
+// rounds: silu is rounded before the product; dg = round(round(dy u) silu'), du = round(dy round(silu)). mode 3: mode 1
+// plus the gradient (cg, cu) that is already there.
 template <typename T, typename A, int MODE>
 __device__ __forceinline__ void glu_elem(A g, A u, A dy, A cg, A cu, T& o0, T& o1, T& o2) {
 #pragma clang fp contract(off)
@@ -218,9 +253,13 @@ __device__ __forceinline__ void glu_elem(A g, A u, A dy, A cg, A cu, T& o0, T& o
         return;
     }
     const A d1 = s * ((A)1 + g * ((A)1 - s));  // silu'
-    if constexpr (MODE == 1) {
+    if constexpr (MODE == 1 || MODE == 3) {
         o0 = narrow<T, A>(wide<T, A>(narrow<T, A>(dy * u)) * d1);
         o1 = narrow<T, A>(dy * wide<T, A>(narrow<T, A>(silu)));
+        if constexpr (MODE == 3) {
+            o0 = add_rounded<T, A>(o0, cg);
+            o1 = add_rounded<T, A>(o1, cu);
+        }
         return;
     }
     const A d2 = s * ((A)1 - s) * ((A)2 + g * ((A)1 - (A)2 * s));  // silu''
@@ -238,12 +277,12 @@ template <typename T, int MODE> __global__ __launch_bounds__(256) void k_swiglu(
         const int j = (int)(e - row * a.I);
         const T* gu = reinterpret_cast<const T*>(a.gu) + row * 2 * a.I;
         const A dy = MODE >= 1 ? wide<T, A>(reinterpret_cast<const T*>(a.dy)[e]) : (A)0;
-        const T* c = MODE == 2 ? reinterpret_cast<const T*>(a.c) + row * 2 * a.I : nullptr;
+        const T* c = MODE >= 2 ? reinterpret_cast<const T*>(a.c) + row * 2 * a.I : nullptr;
         T o0, o1, o2;
-        glu_elem<T, A, MODE>(wide<T, A>(gu[j]), wide<T, A>(gu[a.I + j]), dy, MODE == 2 ? wide<T, A>(c[j]) : (A)0,
-                             MODE == 2 ? wide<T, A>(c[a.I + j]) : (A)0, o0, o1, o2);
+        glu_elem<T, A, MODE>(wide<T, A>(gu[j]), wide<T, A>(gu[a.I + j]), dy, MODE >= 2 ? wide<T, A>(c[j]) : (A)0,
+                             MODE >= 2 ? wide<T, A>(c[a.I + j]) : (A)0, o0, o1, o2);
         if constexpr (MODE == 0) reinterpret_cast<T*>(a.y)[e] = o0;
-        if constexpr (MODE == 1) {
+        if constexpr (MODE == 1 || MODE == 3) {
             T* out = reinterpret_cast<T*>(a.y) + row * 2 * a.I;
             out[j] = o0;
             out[a.I + j] = o1;
@@ -271,7 +310,7 @@ template <typename T, int MODE, typename IDX> __global__ __launch_bounds__(256) 
         const Vec<T> gv = ldv(gu), uv = ldv(gu + I);
         Vec<T> dyv, cgv, cuv, r0, r1, r2;
         if constexpr (MODE >= 1) dyv = ldv(reinterpret_cast<const T*>(a.dy) + (int64_t)v * VEC);
-        if constexpr (MODE == 2) {
+        if constexpr (MODE >= 2) {
             const T* c = reinterpret_cast<const T*>(a.c) + (int64_t)row * 2 * I + j;
             cgv = ldv(c);
             cuv = ldv(c + I);
@@ -279,11 +318,11 @@ template <typename T, int MODE, typename IDX> __global__ __launch_bounds__(256) 
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
             glu_elem<T, A, MODE>(wide<T, A>(gv.e[e]), wide<T, A>(uv.e[e]), MODE >= 1 ? wide<T, A>(dyv.e[e]) : (A)0,
-                                 MODE == 2 ? wide<T, A>(cgv.e[e]) : (A)0, MODE == 2 ? wide<T, A>(cuv.e[e]) : (A)0,
+                                 MODE >= 2 ? wide<T, A>(cgv.e[e]) : (A)0, MODE >= 2 ? wide<T, A>(cuv.e[e]) : (A)0,
                                  r0.e[e], r1.e[e], r2.e[e]);
         if constexpr (MODE == 0) stv(reinterpret_cast<T*>(a.y) + (int64_t)v * VEC, r0);
         if constexpr (MODE >= 1) {
-            T* out = reinterpret_cast<T*>(MODE == 1 ? a.y : a.ggu) + (int64_t)row * 2 * I + j;
+            T* out = reinterpret_cast<T*>(MODE == 2 ? a.ggu : a.y) + (int64_t)row * 2 * I + j;
             stv(out, r0);
             stv(out + I, r1);
         }
@@ -330,8 +369,9 @@ template <typename T, int MODE> static void launch_norm_t(hipStream_t s, const N
 }
 
 template <int MODE> static void launch_norm(int dtype, hipStream_t s, const NormArgs& a) {
-    const bool vec_ok = aligned16(a.x) && (MODE < 1 || aligned16(a.dy)) && (MODE < 2 || aligned16(a.c)) &&
-                        (MODE == 2 ? aligned16(a.gx) && aligned16(a.gdy) : aligned16(a.y));
+    const bool vec_ok = aligned16(a.x) && (MODE < 1 || aligned16(a.dy)) &&
+                        ((MODE != 2 && MODE != 3) || aligned16(a.c)) && (MODE == 2 || aligned16(a.y)) &&
+                        ((MODE != 2 && MODE != 4) || aligned16(a.gx)) && (MODE != 2 || aligned16(a.gdy));
     if (dtype == EBR_DTYPE_F32) launch_norm_t<float, MODE>(s, a, vec_ok);
     else if (dtype == EBR_DTYPE_BF16) launch_norm_t<__bf16, MODE>(s, a, vec_ok);
     else if (dtype == EBR_DTYPE_F16) launch_norm_t<_Float16, MODE>(s, a, vec_ok);
@@ -390,6 +430,26 @@ int ebr_block_rmsnorm_bwd(int dtype, int64_t rows, int C, float eps, const void*
     return rc_launch();
 }
 
+int ebr_block_rmsnorm_bwd_add(int dtype, int64_t rows, int C, float eps, const void* x, const void* dy,
+                              const void* acc, void* dx, void* stream) {
+    int rc = check(dtype, rows, C);
+    if (rc) return rc;
+    if (!x || !dy || !acc || !dx) return EBR_ERR_NULL;
+    NormArgs a = {x, dy, acc, dx, nullptr, nullptr, rows, C, eps};
+    launch_norm<3>(dtype, (hipStream_t)stream, a);
+    return rc_launch();
+}
+
+int ebr_block_add_rmsnorm(int dtype, int64_t rows, int C, float eps, const void* x, const void* r, void* sum, void* y,
+                          void* stream) {
+    int rc = check(dtype, rows, C);
+    if (rc) return rc;
+    if (!x || !r || !sum || !y) return EBR_ERR_NULL;
+    NormArgs a = {x, r, nullptr, y, sum, nullptr, rows, C, eps};
+    launch_norm<4>(dtype, (hipStream_t)stream, a);
+    return rc_launch();
+}
+
 int ebr_block_rmsnorm_bwd2(int dtype, int64_t rows, int C, float eps, const void* x, const void* dy, const void* c,
                            void* gx, void* gdy, void* stream) {
     int rc = check(dtype, rows, C);
@@ -415,6 +475,16 @@ int ebr_block_swiglu_bwd(int dtype, int64_t rows, int I, const void* gu, const v
     if (!gu || !dy || !dgu) return EBR_ERR_NULL;
     GluArgs a = {gu, dy, nullptr, dgu, nullptr, nullptr, rows, I};
     launch_glu<1>(dtype, (hipStream_t)stream, a);
+    return rc_launch();
+}
+
+int ebr_block_swiglu_bwd_add(int dtype, int64_t rows, int I, const void* gu, const void* dy, const void* acc,
+                             void* dgu, void* stream) {
+    int rc = check(dtype, rows, I);
+    if (rc) return rc;
+    if (!gu || !dy || !acc || !dgu) return EBR_ERR_NULL;
+    GluArgs a = {gu, dy, acc, dgu, nullptr, nullptr, rows, I};
+    launch_glu<3>(dtype, (hipStream_t)stream, a);
     return rc_launch();
 }
 

@@ -401,14 +401,36 @@ Tensor rmsnorm(const Tensor& x_, double eps) {
     return y;
 }
 
-Tensor rmsnorm_bwd(const Tensor& x_, const Tensor& dy_, double eps) {
+// {sum, rms_norm(sum)} of sum = a + b
+variable_list add_rmsnorm(const Tensor& a_, const Tensor& b_, double eps) {
+    RECORD_FUNCTION("ebr_fused::block_add_rmsnorm", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(a_.device());
+    const Tensor a = dense(a_), b = dense(b_), sum = at::empty(a.sizes(), a.options());
+    const Tensor y = at::empty(a.sizes(), a.options());
+    const RowsOf r(a);
+    check(ebr_block_add_rmsnorm(dtype_code(a.scalar_type()), r.rows, (int)r.width, (float)eps, a.data_ptr(),
+                                b.data_ptr(), sum.data_ptr(), y.data_ptr(), stream_of(a)),
+          "ebr_block_add_rmsnorm");
+    return {sum, y};
+}
+
+// ``acc``: a gradient of x that is already there and is added, or undefined.
+Tensor rmsnorm_bwd(const Tensor& x_, const Tensor& dy_, const Tensor& acc_, double eps) {
     RECORD_FUNCTION("ebr_fused::block_rmsnorm_bwd", std::vector<c10::IValue>());
     const c10::DeviceGuard on(x_.device());
-    const Tensor x = dense(x_), dy = dense(dy_.to(x_.scalar_type())), dx = at::empty(x.sizes(), x.options());
+    const auto st = x_.scalar_type();
+    const Tensor x = dense(x_), dy = dense(dy_.to(st)), dx = at::empty(x.sizes(), x.options());
     const RowsOf r(x);
-    check(ebr_block_rmsnorm_bwd(dtype_code(x.scalar_type()), r.rows, (int)r.width, (float)eps, x.data_ptr(),
-                                dy.data_ptr(), dx.data_ptr(), stream_of(x)),
-          "ebr_block_rmsnorm_bwd");
+    if (acc_.defined()) {
+        const Tensor acc = dense(acc_.to(st));
+        check(ebr_block_rmsnorm_bwd_add(dtype_code(st), r.rows, (int)r.width, (float)eps, x.data_ptr(), dy.data_ptr(),
+                                        acc.data_ptr(), dx.data_ptr(), stream_of(x)),
+              "ebr_block_rmsnorm_bwd_add");
+    } else {
+        check(ebr_block_rmsnorm_bwd(dtype_code(st), r.rows, (int)r.width, (float)eps, x.data_ptr(), dy.data_ptr(),
+                                    dx.data_ptr(), stream_of(x)),
+              "ebr_block_rmsnorm_bwd");
+    }
     return dx;
 }
 
@@ -430,7 +452,7 @@ struct RmsNormBwd : Function<RmsNormBwd> {
         ctx->save_for_backward({x, dy});
         ctx->saved_data["eps"] = eps;
         ctx->set_materialize_grads(false);
-        return {rmsnorm_bwd(x, dy, eps)};
+        return {rmsnorm_bwd(x, dy, Tensor(), eps)};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return variable_list(3);
@@ -443,17 +465,44 @@ struct RmsNormBwd : Function<RmsNormBwd> {
     }
 };
 
+// The input of a forward node as an output of its own, which the backward's node reads: the gradients that arise there
+// (the second derivative's) then come back to the forward node, whose own gradient kernel adds them.
+Tensor own_input(const Tensor& x) { return x.detach(); }
+
+// The gradient of a norm's input: from dy through the backward's node, plus ``acc``.
+Tensor norm_grad(const Tensor& x, const Tensor& dy, const Tensor& acc, double eps) {
+    if (!dy.defined()) return acc;
+    if (acc.defined() && !at::GradMode::is_enabled()) return rmsnorm_bwd(x, dy, acc, eps);
+    const Tensor dx = RmsNormBwd::apply(x, dy, eps)[0];
+    return acc.defined() ? dx + acc : dx;
+}
+
 struct RmsNorm : Function<RmsNorm> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, double eps) {
-        ctx->save_for_backward({x});
+        const Tensor own = own_input(x);
+        ctx->save_for_backward({own});
         ctx->saved_data["eps"] = eps;
         ctx->set_materialize_grads(false);
-        return {rmsnorm(x, eps)};
+        return {rmsnorm(x, eps), own};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-        if (!g[0].defined()) return variable_list(2);
         const Tensor x = ctx->get_saved_variables()[0];
-        return {RmsNormBwd::apply(x, g[0], ctx->saved_data["eps"].toDouble())[0], Tensor()};
+        return {norm_grad(x, g[0], g[1], ctx->saved_data["eps"].toDouble()), Tensor()};
+    }
+};
+
+struct AddRmsNorm : Function<AddRmsNorm> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& a, const Tensor& b, double eps) {
+        variable_list out = add_rmsnorm(a, b, eps);
+        ctx->save_for_backward({out[0]});
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        return {out[1], out[0]};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        const Tensor x = ctx->get_saved_variables()[0];
+        const Tensor d = norm_grad(x, g[0], g[1], ctx->saved_data["eps"].toDouble());
+        return {d, d, Tensor()};
     }
 };
 
@@ -471,11 +520,19 @@ Tensor swiglu_fwd(const Tensor& gu_) {
     return y;
 }
 
-Tensor swiglu_bwd(const Tensor& gu_, const Tensor& dy_) {
+// ``acc``: a gradient of gu that is already there and is added, or undefined.
+Tensor swiglu_bwd(const Tensor& gu_, const Tensor& dy_, const Tensor& acc_) {
     RECORD_FUNCTION("ebr_fused::block_swiglu_bwd", std::vector<c10::IValue>());
     const c10::DeviceGuard on(gu_.device());
     const Tensor gu = dense(gu_), dy = dense(dy_.to(gu_.scalar_type())), d = at::empty(gu.sizes(), gu.options());
     const RowsOf r(gu);
+    if (acc_.defined()) {
+        const Tensor acc = dense(acc_.to(gu.scalar_type()));
+        check(ebr_block_swiglu_bwd_add(dtype_code(gu.scalar_type()), r.rows, (int)(r.width / 2), gu.data_ptr(),
+                                       dy.data_ptr(), acc.data_ptr(), d.data_ptr(), stream_of(gu)),
+              "ebr_block_swiglu_bwd_add");
+        return d;
+    }
     check(ebr_block_swiglu_bwd(dtype_code(gu.scalar_type()), r.rows, (int)(r.width / 2), gu.data_ptr(), dy.data_ptr(),
                                d.data_ptr(), stream_of(gu)),
           "ebr_block_swiglu_bwd");
@@ -499,7 +556,7 @@ struct SwiGLUBwd : Function<SwiGLUBwd> {
     static variable_list forward(AutogradContext* ctx, const Tensor& gu, const Tensor& dy) {
         ctx->save_for_backward({gu, dy});
         ctx->set_materialize_grads(false);
-        return {swiglu_bwd(gu, dy)};
+        return {swiglu_bwd(gu, dy, Tensor())};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return variable_list(2);
@@ -511,13 +568,17 @@ struct SwiGLUBwd : Function<SwiGLUBwd> {
 
 struct SwiGLU : Function<SwiGLU> {
     static variable_list forward(AutogradContext* ctx, const Tensor& gu) {
-        ctx->save_for_backward({gu});
+        const Tensor own = own_input(gu);
+        ctx->save_for_backward({own});
         ctx->set_materialize_grads(false);
-        return {swiglu_fwd(gu)};
+        return {swiglu_fwd(gu), own};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-        if (!g[0].defined()) return variable_list(1);
-        return SwiGLUBwd::apply(ctx->get_saved_variables()[0], g[0]);
+        if (!g[0].defined()) return {g[1]};
+        const Tensor gu = ctx->get_saved_variables()[0];
+        if (g[1].defined() && !at::GradMode::is_enabled()) return {swiglu_bwd(gu, g[0], g[1])};
+        const Tensor d = SwiGLUBwd::apply(gu, g[0])[0];
+        return {g[1].defined() ? d + g[1] : d};
     }
 };
 
@@ -529,13 +590,20 @@ bool block_takes(const Tensor& x) {
 py::object rms_norm(const py::handle& hx, double eps) {
     const Tensor x = plain(hx);
     if (!block_takes(x)) return py::none();
-    return py::cast(RmsNorm::apply(x, eps)[0]);
+    return py::cast(recorded({x}) ? RmsNorm::apply(x, eps)[0] : rmsnorm(x, eps));
+}
+
+// rms_norm(a + b)
+py::object add_rms_norm(const py::handle& ha, const py::handle& hb, double eps) {
+    const Tensor a = plain(ha), b = plain(hb);
+    if (!block_takes(a) || !b.defined() || a.sizes() != b.sizes() || !same_kind(a, b)) return py::none();
+    return py::cast(recorded({a, b}) ? AddRmsNorm::apply(a, b, eps)[0] : add_rmsnorm(a, b, eps)[1]);
 }
 
 py::object swiglu(const py::handle& hgu) {
     const Tensor gu = plain(hgu);
     if (!block_takes(gu) || gu.size(-1) % 2) return py::none();
-    return py::cast(SwiGLU::apply(gu)[0]);
+    return py::cast(recorded({gu}) ? SwiGLU::apply(gu)[0] : swiglu_fwd(gu));
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -771,6 +839,7 @@ PYBIND11_MODULE(ebr_host, m) {
     m.def("attention", &attention);
     m.def("rope_split", &rope_split);
     m.def("rms_norm", &rms_norm);
+    m.def("add_rms_norm", &add_rms_norm);
     m.def("swiglu", &swiglu);
     m.def("noisy_point", &noisy_point);
     m.def("step_and_project", &step_and_project);

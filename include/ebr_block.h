@@ -24,6 +24,14 @@ int ebr_block_rmsnorm(int dtype, int64_t rows, int C, float eps, const void* x, 
 int ebr_block_rmsnorm_bwd(int dtype, int64_t rows, int C, float eps, const void* x, const void* dy, void* dx,
                           void* stream);
 
+/* As ebr_block_rmsnorm_bwd, plus a gradient that is already there: dx = round(round(dx) + acc). */
+int ebr_block_rmsnorm_bwd_add(int dtype, int64_t rows, int C, float eps, const void* x, const void* dy,
+                              const void* acc, void* dx, void* stream);
+
+/* The residual sum and its norm: sum = round(x + r), y = rms_norm(sum). */
+int ebr_block_add_rmsnorm(int dtype, int64_t rows, int C, float eps, const void* x, const void* r, void* sum, void* y,
+                          void* stream);
+
 /* Gradients of <c, dx> with respect to x (gx) and dy (gdy), dx being ebr_block_rmsnorm_bwd's output. */
 int ebr_block_rmsnorm_bwd2(int dtype, int64_t rows, int C, float eps, const void* x, const void* dy, const void* c,
                            void* gx, void* gdy, void* stream);
@@ -34,6 +42,10 @@ int ebr_block_swiglu(int dtype, int64_t rows, int I, const void* gu, void* y, vo
 
 /* dgu = [dgate | dup] of y given dy. */
 int ebr_block_swiglu_bwd(int dtype, int64_t rows, int I, const void* gu, const void* dy, void* dgu, void* stream);
+
+/* As ebr_block_swiglu_bwd, plus a gradient that is already there: dgu = round(round(dgu) + acc). */
+int ebr_block_swiglu_bwd_add(int dtype, int64_t rows, int I, const void* gu, const void* dy, const void* acc,
+                             void* dgu, void* stream);
 
 /* Gradients of <c, dgu> with respect to gu (ggu, rows of 2 I) and dy (gdy, rows of I). */
 int ebr_block_swiglu_bwd2(int dtype, int64_t rows, int I, const void* gu, const void* dy, const void* c, void* ggu,

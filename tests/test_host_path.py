@@ -92,6 +92,30 @@ def test_same_bits_as_the_python_nodes(monkeypatch, kind, dtype, shape, extra):
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [BF16, F16, F32, torch.float64])
+@pytest.mark.parametrize("shape", [(3, 512), (7, 27), (5, 1032), (2, 2, 4104), (9, 8)])
+@pytest.mark.parametrize("kind", ["norm", "add_norm", "swiglu"])
+def test_sums_inside_the_kernels_round_as_their_own(monkeypatch, kind, shape, dtype):
+    """The residual sum and the second derivative's gradient sums, folded into the norm's and SwiGLU's kernels, against
+    kernels of their own; row widths of every variant (vectors in registers, streamed, odd)."""
+    shape = (*shape[:-1], 2 * shape[-1]) if kind == "swiglu" else shape
+    x, r = (_randn(shape, dtype, i) for i in range(2))
+    out = (*shape[:-1], shape[-1] // 2) if kind == "swiglu" else shape
+
+    def go():
+        # squared, so that the second derivative reaches the forward's node both ways
+        if kind == "norm":
+            return _second_order(lambda a: block.rms_norm(a, 1e-5).square(), [x], [_randn(out, dtype, 3)])
+        if kind == "add_norm":
+            return _second_order(lambda a, b: block.add_rms_norm(a, b, 1e-5).square(), [x, r], [_randn(out, dtype, 3)])
+        return _second_order(lambda a: block.swiglu(a).square(), [x], [_randn(out, dtype, 3)])
+
+    got = go()
+    monkeypatch.setattr(_host, "module", lambda: None)
+    _same(got, go())
+
+
+@gpu
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("per_row,masked", [(True, True), (False, False), (True, False)])
 def test_descent_same_bits_as_the_python_nodes(monkeypatch, dtype, per_row, masked):
@@ -131,6 +155,7 @@ def test_a_single_used_gradient_and_unused_outputs(monkeypatch):
 @gpu
 def test_plain_calls_take_it():
     q = _randn((1, 2, 16, 16), BF16, 0).requires_grad_(True)
+    assert "CppNode" in block.add_rms_norm(q, q, 1e-5).grad_fn.name()
     x = _randn((1, 4, 24), BF16, 0).requires_grad_(True)
     rope = RotaryTable2D(4, 2, 2).cuda()
     for y in (fused_attention(q, q, q), block.rms_norm(q, 1e-5), block.swiglu(q), linear.linear(q, q[0, 0]),
