@@ -91,6 +91,15 @@ SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_int] * 5 + [_P, _I64P] * 3 + [_F32P] * 3 + [_P, _P],
     ),
+    "ebr_rope_graded_scratch": (ctypes.c_int64, [ctypes.c_int] * 5),
+    "ebr_rope_split_graded": (
+        ctypes.c_int,
+        [ctypes.c_int] * 5 + [_P, ctypes.c_int64, ctypes.c_int64] + [_F32P] * 3 + [_P] * 4 + [_F32P] * 2 + [_P],
+    ),
+    "ebr_rope_merge_graded": (
+        ctypes.c_int,
+        [ctypes.c_int] * 5 + [_P, _I64P] * 3 + [_P] * 3 + [_F32P] * 3 + [_P] * 2 + [_F32P] * 2 + [_P],
+    ),
     # include/ebr_descent.h
     "ebr_descent_noisy_point": (
         ctypes.c_int,

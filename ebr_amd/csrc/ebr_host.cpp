@@ -269,7 +269,7 @@ py::object attention(const py::handle& hq, const py::handle& hk, const py::handl
     if (code < 0 || code == EBR_DTYPE_F64 || q.numel() == 0) return py::none();
     const int64_t D = q.size(3);
     if (D > 256 || D % (code == EBR_DTYPE_F32 ? 4 : 8) || q.numel() / D >= (int64_t(1) << 31)) return py::none();
-    return py::cast(AttnFwd::apply(q, k, v, scale ? *scale : 1.0 / std::sqrt((double)D))[0]);
+    return py::cast(AttnFwd::apply(q, k, v, scale ? *scale : std::pow((double)D, -0.5))[0]);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -377,6 +377,186 @@ py::object rope_split(const py::handle& hqkv, const py::handle& hcos, const py::
     sin = sin.to(at::kFloat).contiguous();
     const variable_list o = RopeSplit::apply(qkv, cos, sin, maybe(qs), heads);
     return py::make_tuple(o[0], o[1], o[2]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Rotary split, temperature, attention and the heads' merge as one node: y [B, N, H D] of a projection qkv [B, N, 3 H D].
+// The split's q (tempered), k and v are outputs of the node that its backward's node reads, so the second derivative's
+// gradients of them come back here and the merge adds them.
+// ---------------------------------------------------------------------------------------------------------------------
+
+Tensor heads_apart(const Tensor& y, int64_t heads) {  // [B, N, H D] as [B, H, N, D]
+    return y.reshape({y.size(0), y.size(1), heads, y.size(2) / heads}).transpose(1, 2);
+}
+
+Tensor heads_together(const Tensor& o) {
+    return o.transpose(1, 2).reshape({o.size(0), o.size(2), o.size(1) * o.size(3)});
+}
+
+Tensor head_scratch(const Tensor& like, int64_t B, int64_t N, int64_t H, int64_t D) {
+    const int64_t n = ebr_rope_graded_scratch(dtype_code(like.scalar_type()), (int)B, (int)N, (int)H, (int)D);
+    return at::empty({n / 4}, like.options().dtype(at::kFloat));
+}
+
+// {q, k, v, dt}: the split of qkv with the temperature t; dt = per-head sums of w and the rotated q where w is defined.
+variable_list split_graded(const Tensor& qkv, const Tensor& cos, const Tensor& sin, const Tensor& t, const Tensor& w,
+                           int64_t heads) {
+    RECORD_FUNCTION("ebr_fused::rope_split", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(qkv.device());
+    const Tensor x = contig(qkv);
+    const int64_t B = x.size(0), N = x.size(1), D = x.size(2) / (3 * heads);
+    variable_list out(4);
+    for (int i = 0; i < 3; ++i) out[i] = at::empty({B, heads, N, D}, x.options());
+    Tensor part;
+    if (w.defined()) {
+        out[3] = at::empty({heads}, t.options());
+        part = head_scratch(x, B, N, heads, D);
+    }
+    check(ebr_rope_split_graded(dtype_code(x.scalar_type()), (int)B, (int)N, (int)heads, (int)D, x.data_ptr(),
+                                x.stride(0), x.stride(1), fptr(cos), fptr(sin), fptr(t), out[0].data_ptr(),
+                                out[1].data_ptr(), out[2].data_ptr(), w.defined() ? w.data_ptr() : nullptr,
+                                fptr(out[3]), fptr(part), stream_of(x)),
+          "ebr_rope_split_graded");
+    return out;
+}
+
+// {g, dt}: the merge of d plus add (three gradients each; add may be undefined); dt where qkv is defined.
+variable_list merge_graded(const Tensor (&d_)[3], const Tensor (&add_)[3], const Tensor& cos, const Tensor& sin,
+                           const Tensor& t, const Tensor& qkv_) {
+    RECORD_FUNCTION("ebr_fused::rope_merge", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(d_[0].device());
+    const auto st = d_[0].scalar_type();
+    Tensor d[3], add[3];
+    for (int i = 0; i < 3; ++i) {
+        d[i] = rows(d_[i].to(st));
+        if (add_[i].defined()) add[i] = contig(add_[i].to(st));
+    }
+    const Dims m(d[0]);
+    const Tensor g = at::empty({m.B, m.L, int64_t(3) * m.H * m.D}, d[0].options());
+    Tensor dt, part, qkv;
+    if (qkv_.defined()) {
+        qkv = contig(qkv_);
+        dt = at::empty({m.H}, t.options());
+        part = head_scratch(d[0], m.B, m.L, m.H, m.D);
+    }
+    const auto ptr = [](const Tensor& x) -> const void* { return x.defined() ? x.data_ptr() : nullptr; };
+    check(ebr_rope_merge_graded(dtype_code(st), m.B, m.H, m.L, m.D, d[0].data_ptr(), Str3(d[0]).s, d[1].data_ptr(),
+                                Str3(d[1]).s, d[2].data_ptr(), Str3(d[2]).s, ptr(add[0]), ptr(add[1]), ptr(add[2]),
+                                fptr(cos), fptr(sin), fptr(t), g.data_ptr(), ptr(qkv), fptr(dt), fptr(part),
+                                stream_of(g)),
+          "ebr_rope_merge_graded");
+    return {g, dt};
+}
+
+// The gradient of qkv from dy as a differentiable node (inputs t, q, k, v, dy; o and lse are constants in it).
+struct RopeAttnBwd : Function<RopeAttnBwd> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& t, const Tensor& q, const Tensor& k,
+                                 const Tensor& v, const Tensor& dy, const Tensor& o, const Tensor& lse,
+                                 const Tensor& cos, const Tensor& sin, double scale) {
+        const variable_list d = attn_bwd(q, k, v, o, lse, heads_apart(dy, q.size(1)), scale);
+        ctx->save_for_backward({t, q, k, v, dy, o, lse, cos, sin, d[0]});
+        ctx->saved_data["scale"] = scale;
+        ctx->set_materialize_grads(false);
+        return {merge_graded({d[0], d[1], d[2]}, {Tensor(), Tensor(), Tensor()}, cos, sin, t, Tensor())[0]};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        variable_list out(10);
+        if (!g[0].defined()) return out;
+        const bool want_t = ctx->needs_input_grad(0);
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &t = s[0], &q = s[1], &dy = s[4];
+        const int64_t heads = q.size(1);
+        const variable_list c = split_graded(g[0].to(q.scalar_type()), s[7], s[8], t, want_t ? s[9] : Tensor(), heads);
+        const variable_list h = attn_bwd_bwd(q, s[2], s[3], s[5], s[6], heads_apart(dy, heads), c[0], c[1], c[2],
+                                             ctx->saved_data["scale"].toDouble());
+        variable_list d = {c[3], h[0], h[1], h[2], heads_together(h[3])};
+        if (recorded({t, q, s[2], s[3], dy, g[0]})) d = last(std::move(d));
+        for (size_t i = 0; i < d.size(); ++i) out[i] = d[i];
+        return out;
+    }
+};
+
+struct RopeAttn : Function<RopeAttn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& t, const Tensor& cos,
+                                 const Tensor& sin, int64_t heads, double scale) {
+        const variable_list x = split_graded(qkv, cos, sin, t, Tensor(), heads);
+        const variable_list o = attn_fwd(x[0], x[1], x[2], scale);
+        ctx->save_for_backward({t.requires_grad() ? qkv : Tensor(), t, cos, sin, x[0], x[1], x[2], o[0], o[1]});
+        ctx->saved_data["scale"] = scale;
+        ctx->set_materialize_grads(false);
+        return {heads_together(o[0]), x[0], x[1], x[2]};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& g) {
+        variable_list out(6);
+        const Tensor& dy = g[0];
+        const bool more = g[1].defined() || g[2].defined() || g[3].defined();
+        if (!dy.defined() && !more) return out;
+        const bool want_t = ctx->needs_input_grad(1);
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &qkv = s[0], &t = s[1], &cos = s[2], &sin = s[3], &q = s[4], &k = s[5], &v = s[6];
+        const int64_t heads = q.size(1);
+        const double scale = ctx->saved_data["scale"].toDouble();
+        if (at::GradMode::is_enabled()) {
+            if (!more && !want_t) {
+                out[0] = RopeAttnBwd::apply(t, q, k, v, dy, s[7], s[8], cos, sin, scale)[0];
+                return out;
+            }
+            // every part as a node of its own, for derivatives of any of them
+            Tensor d[3];
+            if (dy.defined()) {
+                const variable_list a = AttnBwd::apply(q, k, v, s[7], s[8], heads_apart(dy, heads), scale);
+                for (int i = 0; i < 3; ++i) d[i] = a[i];
+            }
+            for (int i = 0; i < 3; ++i) {
+                if (g[i + 1].defined()) d[i] = d[i].defined() ? d[i] + g[i + 1] : g[i + 1];
+                if (!d[i].defined()) d[i] = at::zeros({q.size(3)}, q.options()).expand(q.sizes());
+            }
+            if (want_t) {
+                const Tensor rq = RopeSplit::apply(qkv, cos, sin, std::nullopt, heads)[0];
+                out[1] = (d[0] * rq).sum({0, 2, 3}, false, at::kFloat).to(t.scalar_type());
+            }
+            const Tensor td = t.to(q.scalar_type()).view({1, heads, 1, 1});
+            out[0] = RopeMerge::apply(d[0] * td, d[1], d[2], cos, sin, std::nullopt)[0];
+            return out;
+        }
+        Tensor d[3], add[3];
+        if (dy.defined()) {
+            const variable_list a = attn_bwd(q, k, v, s[7], s[8], heads_apart(dy, heads), scale);
+            for (int i = 0; i < 3; ++i) {
+                d[i] = a[i];
+                if (more) add[i] = g[i + 1].defined() ? g[i + 1] : at::zeros_like(q);
+            }
+        } else {
+            for (int i = 0; i < 3; ++i)
+                d[i] = g[i + 1].defined() ? g[i + 1] : at::zeros({q.size(3)}, q.options()).expand(q.sizes());
+        }
+        const variable_list m = merge_graded(d, add, cos, sin, t, want_t ? qkv : Tensor());
+        out[0] = m[0];
+        out[1] = m[1];
+        return out;
+    }
+};
+
+// Attention of a projection with the rotary tables and the temperature ``ht`` (fp32 [H], rounded to the dtype inside).
+py::object rope_attention(const py::handle& hqkv, const py::handle& hcos, const py::handle& hsin, int64_t heads,
+                          const py::handle& ht) {
+    const Tensor qkv = plain(hqkv), cos = plain(hcos), sin = plain(hsin), t = plain(ht);
+    if (!qkv.defined() || !cos.defined() || !sin.defined() || !t.defined() || !plain_context()) return py::none();
+    const int code = dtype_code(qkv.scalar_type());
+    if (code < 0 || code == EBR_DTYPE_F64 || heads < 1 || qkv.dim() != 3 || qkv.numel() == 0 ||
+        qkv.size(2) % (3 * heads))
+        return py::none();
+    const int64_t B = qkv.size(0), N = qkv.size(1), D = qkv.size(2) / (3 * heads);
+    const std::vector<int64_t> table = {N, D};
+    if (D > 128 || cos.sizes() != table || sin.sizes() != table || t.dim() != 1 || t.size(0) != heads ||
+        B * heads * N >= (int64_t(1) << 31))
+        return py::none();
+    for (const Tensor& x : {cos, sin, t})
+        if (x.scalar_type() != at::kFloat || !x.is_contiguous() || x.device() != qkv.device() ||
+            reinterpret_cast<uintptr_t>(x.data_ptr()) % (x.dim() == 2 ? 32 : 4))
+            return py::none();
+    if (ebr_rope_graded_scratch(code, (int)B, (int)N, (int)heads, (int)D) == 0) return py::none();
+    return py::cast(RopeAttn::apply(qkv, t, cos, sin, heads, std::pow((double)D, -0.5))[0]);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -838,6 +1018,7 @@ PYBIND11_MODULE(ebr_host, m) {
         throw std::runtime_error("libebr_attn.so has another ABI version than this module was built for");
     m.def("attention", &attention);
     m.def("rope_split", &rope_split);
+    m.def("rope_attention", &rope_attention);
     m.def("rms_norm", &rms_norm);
     m.def("add_rms_norm", &add_rms_norm);
     m.def("swiglu", &swiglu);

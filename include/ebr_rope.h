@@ -39,6 +39,26 @@ int ebr_rope_merge(int dtype, int B, int H, int N, int D, const void* dq, const 
                    const int64_t dk_str[3], const void* dv, const int64_t dv_str[3], const float* cos,
                    const float* sin, const float* qscale, void* g, void* stream);
 
+/* Bytes of fp32 scratch that the per-head sums of the two entries below need; 0 for a dtype, size or head dim that they do
+ * not take (D must hold a power of two, at most 64, of 16-byte vectors, and a quarter of D whole vectors). */
+int64_t ebr_rope_graded_scratch(int dtype, int B, int N, int H, int D);
+
+/* ebr_rope_split with the learned temperature t (fp32 [H], rounded to the dtype here), and, where w ([B, H, N, D],
+ * contiguous, 16-byte aligned) is given, dt[h] = sum over head h of w * R q (products and sum
+ * rounded to the dtype, the sum taken in fp32), R q the rotated and rounded q before the
+ * temperature. All pointers and row starts 16-byte aligned (else EBR_ERR_ALIGN, nothing enqueued). */
+int ebr_rope_split_graded(int dtype, int B, int N, int H, int D, const void* qkv, int64_t qkv_sb, int64_t qkv_sn,
+                          const float* cos, const float* sin, const float* t, void* q, void* k, void* v,
+                          const void* w, float* dt, float* scratch, void* stream);
+
+/* Its adjoint: ebr_rope_merge of dq + aq, dk + ak, dv + av (each sum rounded to the dtype; aq, ak, av contiguous
+ * [B, H, N, D], or all NULL), and, where qkv (the split's contiguous input) is given, dt[h] = sum over head h of
+ * (dq + aq) * R q. */
+int ebr_rope_merge_graded(int dtype, int B, int H, int N, int D, const void* dq, const int64_t dq_str[3],
+                          const void* dk, const int64_t dk_str[3], const void* dv, const int64_t dv_str[3],
+                          const void* aq, const void* ak, const void* av, const float* cos, const float* sin,
+                          const float* t, void* g, const void* qkv, float* dt, float* scratch, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

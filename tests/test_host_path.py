@@ -273,3 +273,74 @@ def test_host_command_links_the_library_beside_it():
 
     cmd = build.host_command(Path("x.so"))
     assert "-lebr_attn" in cmd and "-Wl,-rpath,$ORIGIN" in cmd and cmd[-1] == "x.so"
+
+
+def _parts(qkv, cos, sin, heads, t):
+    """rope_attention by its parts."""
+    b, n, _ = qkv.shape
+    q, k, v = rope_split(qkv, cos, sin, heads)
+    y = fused_attention(q * t.to(q.dtype).view(1, heads, 1, 1), k, v)
+    return y.transpose(1, 2).reshape(b, n, -1)
+
+
+def _close(got, want, dtype, size):
+    """Bits for what the parts round alike; the temperature's gradient to its sum's precision: the parts round every
+    product and their sum to the dtype, an error of a few roundings of the products' 2-norm (``size``)."""
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is None:
+            continue
+        if a.dim() == 1:
+            scale = b.float().abs().max().clamp_min(size)
+            assert ((a.float() - b.float()).abs().max() / scale).item() < {BF16: 3e-2, F16: 4e-3, F32: 1e-5}[dtype]
+        else:
+            assert torch.equal(a, b)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [BF16, F16, F32])
+@pytest.mark.parametrize("B,grid,H,D", [(1, (3, 3), 1, 32), (3, (3, 5), 3, 64), (5, (7, 7), 4, 128), (2, (12, 12), 8, 32)])
+def test_rope_attention_is_its_parts(dtype, B, grid, H, D):
+    """Rows that fill no workgroup and rows that fill many; heads that no workgroup holds evenly."""
+    from ebr_amd.fused_attn.rope_split import rope_attention
+
+    N = grid[0] * grid[1]
+    cos, sin = RotaryTable2D(D, *grid).cuda()()
+    qkv, dy, c = _randn((B, N, 3 * H * D), dtype, 1), _randn((B, N, H * D), dtype, 2), _randn((B, N, 3 * H * D), dtype, 3)
+    t0 = torch.linspace(0.7, 1.6, H, device="cuda")
+
+    def go(fn):
+        x, t, d = qkv.clone().requires_grad_(True), t0.clone().requires_grad_(True), dy.clone().requires_grad_(True)
+        y = fn(x, cos, sin, H, t)
+        assert y is not None
+        (g,) = torch.autograd.grad(y, x, d, create_graph=True)
+        second = torch.autograd.grad(g, (x, t, d), c, retain_graph=True)  # nothing uses y a second time
+        both = torch.autograd.grad([g, y.float().square().to(dtype)], (x, t), [c, dy], retain_graph=True)
+        gt = torch.autograd.grad(y, (x, t), dy, create_graph=True)  # every part recorded
+        third = torch.autograd.grad(gt[0], (x, t), c)
+        plain = torch.autograd.grad(fn(x, cos, sin, H, t.detach()), x, dy)  # an inference step
+        return [y, g, *second, *both, *gt, *third, *plain]
+
+    got, want = go(rope_attention), go(_parts)
+    # a head's products dq * R q as independent values of the norms of g and qkv
+    size = (want[1].float().norm() * qkv.float().norm() / (3 * H * (B * N * D) ** 0.5)).item()
+    _close(got, want, dtype, size)
+    assert torch.equal(go(rope_attention)[3], got[3])  # the same sums on every run
+
+
+@gpu
+def test_rope_attention_leaves_other_calls():
+    from ebr_amd.fused_attn.rope_split import rope_attention
+
+    t = torch.ones(2, device="cuda")
+    for D in (16, 96, 20):  # no power of two of whole vectors
+        cos, sin = RotaryTable2D(D, 2, 2).cuda()()
+        assert rope_attention(_randn((1, 4, 6 * D), BF16, 0), cos, sin, 2, t) is None
+    cos, sin = RotaryTable2D(32, 2, 2).cuda()()
+    x = _randn((1, 4, 192), BF16, 0)
+    assert rope_attention(x, cos, sin, 2, torch.ones(3, device="cuda")) is None
+    assert rope_attention(x, cos, sin, 2, t.bfloat16()) is None and rope_attention(x, cos[1:], sin, 2, t) is None
+    assert rope_attention(x.double(), cos, sin, 2, t) is None
+    with _Seen() as seen:
+        assert rope_attention(x, cos, sin, 2, t) is None
+    assert not seen.ops
