@@ -130,6 +130,7 @@ SIGNATURES = {
     "ebr_block_swiglu_bwd": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 4),
     "ebr_block_swiglu_bwd_add": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 5),
     "ebr_block_swiglu_bwd2": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int] + [_P] * 6),
+    "ebr_block_split_sum": (ctypes.c_int, [ctypes.c_int] * 2 + [ctypes.c_int64, _F32P, _P, _P]),
     "ebr_attn_error_string": (ctypes.c_char_p, [ctypes.c_int]),
     "ebr_attn_abi_version": (ctypes.c_int, []),
     "ebr_attn_arch": (ctypes.c_char_p, []),

@@ -961,7 +961,12 @@ Tensor weight_grad(const Tensor& a, const Tensor& b) {
     if (s == 1) return at::matmul(a2.t(), b2);
     const Tensor a3 = a2.contiguous().view({s, m / s, n}).transpose(1, 2);
     const Tensor b3 = b2.contiguous().view({s, m / s, k});  // the right operand stays a contiguous batch
-    return at::bmm(a3, b3, at::kFloat).sum(0).to(a.scalar_type());
+    const Tensor part = at::bmm(a3, b3, at::kFloat);
+    const c10::DeviceGuard on(a.device());
+    const Tensor out = at::empty({n, k}, a2.options().requires_grad(false));
+    check(ebr_block_split_sum(dtype_code(a.scalar_type()), (int)s, n * k, fptr(part), out.data_ptr(), stream_of(a)),
+          "ebr_block_split_sum");
+    return out;
 }
 
 struct Linear;

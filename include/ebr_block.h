@@ -51,6 +51,9 @@ int ebr_block_swiglu_bwd_add(int dtype, int64_t rows, int I, const void* gu, con
 int ebr_block_swiglu_bwd2(int dtype, int64_t rows, int I, const void* gu, const void* dy, const void* c, void* ggu,
                           void* gdy, void* stream);
 
+/* out[i] = round(sum over s of part[s][i]) of S (2, 4, 8 or 16) fp32 partial products [S, n]; out in bf16 or fp16. */
+int ebr_block_split_sum(int dtype, int S, int64_t n, const float* part, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -116,6 +116,20 @@ def test_sums_inside_the_kernels_round_as_their_own(monkeypatch, kind, shape, dt
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("rows,N,K", [(2048, 48, 32), (4096, 7, 9), (8192, 40, 24), (16384, 33, 65), (16384, 256, 6144)])
+def test_split_weight_gradients(dtype, rows, N, K):
+    """2, 4, 8 and 16 partial products (8 where the output is large), whole vectors and odd sizes."""
+    x, dy = _randn((rows, K), dtype, 1), _randn((rows, N), dtype, 2)
+    w = _randn((N, K), dtype, 3).requires_grad_(True)
+    (got,) = torch.autograd.grad(linear.linear(x, w), w, dy)
+    want = dy.double().t() @ x.double()
+    # fp32 sums of exact products, rounded once: half an ulp of the dtype, plus the sums' own error
+    eps = torch.finfo(dtype).eps
+    assert ((got.double() - want).abs() <= 0.51 * eps * want.abs() + 1e-5 * rows**0.5).all()
+
+
+@gpu
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("per_row,masked", [(True, True), (False, False), (True, False)])
 def test_descent_same_bits_as_the_python_nodes(monkeypatch, dtype, per_row, masked):
