@@ -1,7 +1,7 @@
 // MFMA fragments, LDS chunk staging and lane reductions for the gfx950 attention kernels.
 //
 // Every contraction in the attention path is written as one of two shapes, both on the 16x16 MFMA tile
-// (v_mfma_f32_16x16x32_{bf16,f16} for 16-bit inputs, v_mfma_f32_16x16x4_f32 for fp32):
+// (v_mfma_f32_16x16x32_{bf16,f16} for 16-bit inputs; for fp32 v_mfma_f32_16x16x4_f32, or the bf16 one on split values):
 //
 //   d-contraction   C[m = x][n = own]  = sum_d X[x][d] * Own[own][d]
 //                   A = rows of the "other side" tensor X from LDS in natural [x][d] layout,
