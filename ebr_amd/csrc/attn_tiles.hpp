@@ -62,9 +62,9 @@ struct f32n {
 // and a plane is read transposed, so a tensor is staged once instead of natural and transposed. Measured at B H = 64,
 // L = 400, D = 64 (fp32 MFMA -> split): forward 41.4 -> 31.9, backward 126 -> 85, bwd_bwd 328 -> 186 us, the error
 // against 64 bits 4.6e-7 -> 3.6e-7, 5.9e-7 -> 5.0e-7, 7.2e-7 -> 6.1e-7 (fewer roundings per sum).
-// Non-finite inputs (and values past bf16's range) do not survive the split: they give NaN wherever they enter, and a
-// workgroup whose outputs hold a NaN computes them again with f32n (see redo_if_nan), so the results for such inputs
-// are those of plain fp32 arithmetic.
+// Non-finite inputs (and values past bf16's range) do not survive the split: they give NaN wherever they enter; and parts
+// below bf16's normal range are taken as zero. A workgroup whose sums hold a NaN or a value below 2^-104 computes them
+// again with f32n (see redo_unsplit), so the results for such inputs are those of plain fp32 arithmetic.
 constexpr int NPLANE = 3;
 
 template <typename T> struct ET;

@@ -103,18 +103,26 @@ __device__ __forceinline__ void store_rows(void* out, int64_t row_off, const f32
 // Forward (row pass): online softmax over 32-key chunks.
 // =====================================================================================================================
 
-// Whether a lane's sums hold a NaN (infinities of both signs count as one).
-template <int N> __device__ __forceinline__ float total(const f32x4 (&v)[N]) {
-    float s = 0.f;
+// Whether a lane's split sums hold a NaN, or a value so small that parts of its terms were subnormal (a bf16 MFMA takes
+// those as zero): below 2^-104, where the smallest parts, 2^-16 of theirs, come within 2^6 of the smallest normal, 2^-126.
+template <typename T> __device__ __forceinline__ bool unsplit(float v) {
+    return ET<T>::SPLIT && !(fabsf(v) >= 0x1p-104f || v == 0.f);
+}
+template <typename T, int N> __device__ __forceinline__ bool unsplit(const f32x4 (&v)[N]) {
+    bool any = false;
+    if constexpr (ET<T>::SPLIT) {
 #pragma unroll
-    for (int t = 0; t < N; ++t) s += (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
-    return s;
+        for (int t = 0; t < N; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) any = any || unsplit<T>(v[t][r]);
+    }
+    return any;
 }
 
-// Runs ``body`` (which returns whether an output row of this lane holds a NaN) with T; split products give NaN for
-// non-finite inputs where fp32 arithmetic may give an infinity, so a workgroup that saw a NaN runs again with f32n,
-// which overwrites everything the first run wrote.
-template <typename T, class Body> __device__ __forceinline__ void redo_if_nan(Body&& body) {
+// Runs ``body`` (which returns whether a sum of this lane is one of those) with T; split products give NaN for
+// non-finite inputs where fp32 arithmetic may give an infinity, and lose bits of values near 2^-126, so a workgroup that
+// saw either runs again with f32n, which overwrites everything the first run wrote.
+template <typename T, class Body> __device__ __forceinline__ void redo_unsplit(Body&& body) {
     const bool bad = body(T{});
     if constexpr (ET<T>::SPLIT) {
         if (__syncthreads_or(bad)) body(f32n{});
@@ -220,19 +228,19 @@ template <typename T, int DP> __device__ __forceinline__ bool fwd_pass(const Arg
     }
     if (!active) return false;
     lsum = xsum4(lsum);
-    const float nan = total(acc) + lsum;
+    const bool redo = unsplit<T>(acc) || unsplit<T>(lsum);
     if (own < L) {
         const int64_t r = (int64_t)bh * L + own;
         store_rows<T, DP>(a.out0, r * D, acc, 1.f / lsum, D, w.g);
         if (w.g == 0) a.lse_out[r] = m + logf(lsum);
     }
-    return own < L && nan != nan;
+    return own < L && redo;
 }
 
 // Wider rows than DP = 128 run 256-thread workgroups (one wave per SIMD, every register for the wave).
 template <typename T, int DP> __global__ __launch_bounds__(DP > 128 ? 256 : 512) void k_fwd(Args a) {
     __shared__ __align__(16) unsigned char smem[FwdSmem<T, DP>::BYTES];
-    redo_if_nan<T>([&](auto t) { return fwd_pass<decltype(t), DP>(a, smem); });
+    redo_unsplit<T>([&](auto t) { return fwd_pass<decltype(t), DP>(a, smem); });
 }
 
 // =====================================================================================================================
@@ -318,10 +326,7 @@ template <typename T, int DP, bool FUSED> struct BwdRow {
 #pragma unroll
         for (int t = 0; t < LY::NT; ++t) acc[t] = mma_seq<T>(acc[t], read_seqa<T, DP>(Kt, t, w.l16, w.g), dsb);
     }
-    __device__ __forceinline__ bool nan(int L) const {
-        const float v = total(acc);
-        return active && own < L && v != v;
-    }
+    __device__ __forceinline__ bool redo(int L) const { return active && own < L && unsplit<T>(acc); }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) store_rows<T, DP>(a.out0, ((int64_t)bh * a.L + own) * a.D, acc, a.scale, a.D, w.g);
     }
@@ -389,9 +394,8 @@ template <typename T, int DP> struct BwdCol {
             ak[t] = mma_seq<T>(ak[t], read_seqa<T, DP>(Qt, t, w.l16, w.g), dsb);
         }
     }
-    __device__ __forceinline__ bool nan(int L) const {
-        const float v = total(ak) + total(av);
-        return active && own < L && v != v;
+    __device__ __forceinline__ bool redo(int L) const {
+        return active && own < L && (unsplit<T>(ak) || unsplit<T>(av));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) {
@@ -529,9 +533,9 @@ template <typename T, int DP, bool FUSED> struct BbRow {
             }
         }
     }
-    __device__ __forceinline__ bool nan(int L) const {
-        const float v = total(X) + total(U) + total(Z) + total(Wv) + e_acc + t_acc;
-        return active && own < L && v != v;
+    __device__ __forceinline__ bool redo(int L) const {
+        return active && own < L &&
+               (unsplit<T>(X) || unsplit<T>(U) || unsplit<T>(Z) || unsplit<T>(Wv) || unsplit<T>(e_acc + t_acc));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w, float* st) {
         const float E = xsum4(e_acc);
@@ -651,9 +655,8 @@ template <typename T, int DP> struct BbCol {
             hv[t] = mma_seq<T>(hv[t], read_seqa<T, DP>(Ot, t, w.l16, w.g), pab);
         }
     }
-    __device__ __forceinline__ bool nan(int L) const {
-        const float v = total(hk) + total(hv);
-        return active && own < L && v != v;
+    __device__ __forceinline__ bool redo(int L) const {
+        return active && own < L && (unsplit<T>(hk) || unsplit<T>(hv));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
         if (active && own < a.L) {
@@ -716,7 +719,7 @@ __device__ __forceinline__ bool fused_two_pass(const Args& a, unsigned char* sme
             cst.load(csrc, 0, L, D, w.tid, w.nthr);
         if constexpr (!LATE) row.chunk(a, x0, smem, w);
     }
-    bool nan = row.nan(L);
+    const bool redo = row.redo(L);
     if constexpr (NSTAT == 1) {
         row.finish(a, w);
     } else {
@@ -732,7 +735,7 @@ __device__ __forceinline__ bool fused_two_pass(const Args& a, unsigned char* sme
         if constexpr (!LATE) col.chunk(a, smem, st + x0, STAT_MAX, w);
     }
     col.finish(a, w);
-    return nan || col.nan(L);
+    return redo || col.redo(L);
 }
 
 template <typename T, int DP> struct FusedSmem {
@@ -745,7 +748,7 @@ template <typename T, int DP> struct FusedSmem {
 template <typename T, int DP> __global__ __launch_bounds__(512) void k_bwd_fused(Args a) {
     __shared__ __align__(16) unsigned char smem[FusedSmem<T, DP>::BWD];
     __shared__ __align__(16) float st[2 * STAT_MAX];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return fused_two_pass<U, DP, BwdRow<U, DP, true>, BwdCol<U, DP>, 2, 1>(a, smem, st);
     });
@@ -754,7 +757,7 @@ template <typename T, int DP> __global__ __launch_bounds__(512) void k_bwd_fused
 template <typename T, int DP> __global__ __launch_bounds__(512) void k_bb_fused(Args a) {
     __shared__ __align__(16) unsigned char smem[FusedSmem<T, DP>::BB];
     __shared__ __align__(16) float st[4 * STAT_MAX];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return fused_two_pass<U, DP, BbRow<U, DP, true>, BbCol<U, DP>, 3, 3>(a, smem, st);
     });
@@ -792,13 +795,13 @@ __device__ __forceinline__ bool stream_row(const Args& a, unsigned char* smem) {
         if (x0 + CH < L) rst.load(src, x0 + CH, L, D, w.tid, w.nthr);
         if constexpr (!LATE) row.chunk(a, x0, smem, w);
     }
-    const bool nan = row.nan(L);
+    const bool redo = row.redo(L);
     if constexpr (BB) {
         row.finish(a, w, nullptr);
     } else {
         row.finish(a, w);
     }
-    return nan;
+    return redo;
 }
 
 // Two-launch col kernel: own rows [blk * 16 W, (blk + 1) * 16 W) of one (b, h); statistics staged from a.lse/a.stats.
@@ -835,12 +838,12 @@ __device__ __forceinline__ bool stream_col(const Args& a, unsigned char* smem) {
         if constexpr (!LATE) col.chunk(a, smem, stc, CH, w);
     }
     col.finish(a, w);
-    return col.nan(L);
+    return col.redo(L);
 }
 
 template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_row(Args a) {
     __shared__ __align__(16) unsigned char smem[BwdRow<T, DP, false>::SMEM];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return stream_row<U, DP, BwdRow<U, DP, false>, 2, false>(a, smem);
     });
@@ -848,7 +851,7 @@ template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_row(A
 
 template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_col(Args a) {
     __shared__ __align__(16) unsigned char smem[BwdCol<T, DP>::SMEM + 2 * CH * 4];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return stream_col<U, DP, BwdCol<U, DP>, 2, 1>(a, smem);
     });
@@ -860,7 +863,7 @@ template <typename T, int DP> __global__ __launch_bounds__(256) void k_bwd_col(A
 
 template <typename T, int DP> __global__ __launch_bounds__(256) BB_SPLIT_WAVES(T, DP) void k_bb_row(Args a) {
     __shared__ __align__(16) unsigned char smem[BbRow<T, DP, false>::SMEM];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return stream_row<U, DP, BbRow<U, DP, false>, 4, true>(a, smem);
     });
@@ -868,7 +871,7 @@ template <typename T, int DP> __global__ __launch_bounds__(256) BB_SPLIT_WAVES(T
 
 template <typename T, int DP> __global__ __launch_bounds__(256) BB_SPLIT_WAVES(T, DP) void k_bb_col(Args a) {
     __shared__ __align__(16) unsigned char smem[BbCol<T, DP>::SMEM + 4 * CH * 4];
-    redo_if_nan<T>([&](auto t) {
+    redo_unsplit<T>([&](auto t) {
         using U = decltype(t);
         return stream_col<U, DP, BbCol<U, DP>, 3, 3>(a, smem);
     });

@@ -75,6 +75,23 @@ def test_non_finite_and_huge_values_as_in_fp32(shape):
     assert torch.isinf(hdo[0, 0, :, 1]).all() and torch.isfinite(hdo[0, 0, :, 2:]).all()
 
 
+@pytest.mark.parametrize("shape", [(1, 2, 140, 64), (1, 1, 50, 32)])
+@pytest.mark.parametrize("size", [1e-30, 1e-36])
+def test_tiny_values_keep_their_precision(shape, size):
+    """Values whose smaller parts fall below bf16's normal range: fp32 carries them, and so does the op."""
+    B, H, L, D = shape
+    q, k, v, do, gq, gk, gv = (t.cuda() for t in oracle.make_inputs(B, H, L, D, dtype=F32, seed=2, qkv_scale=0.5))
+    scale = D**-0.5
+    o, lse = ops._hip_fwd(q, k, v * size, scale)
+    p = torch.softmax(q.cpu().double() @ k.cpu().double().transpose(-1, -2) * scale, dim=-1)
+    want = p @ (v * size).cpu().double()
+    assert ((o.cpu().double() - want).norm() / want.norm()).item() < 1.5e-6
+    o, lse = ops._hip_fwd(q, k, v, scale)
+    dv = ops._hip_bwd(q, k, v, o, lse, do * size, scale)[2].cpu().double()
+    want = p.transpose(-1, -2) @ (do * size).cpu().double()
+    assert ((dv - want).norm() / want.norm()).item() < 1.5e-6
+
+
 def test_repeated_calls_give_the_same_bits():
     ts = [t.cuda() for t in oracle.make_inputs(2, 2, 200, 64, dtype=F32, seed=4, qkv_scale=0.5)]
     first = _run(*ts, 0.125)
