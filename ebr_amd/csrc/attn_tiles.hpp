@@ -21,6 +21,7 @@
 // neutralise (scores of padded keys).
 #pragma once
 
+#include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -54,18 +55,25 @@ struct f32n {
     __device__ operator float() const { return v; }
 };
 
-// Split products. x = hi + mid + lo with each part x's remainder rounded to bf16 (8 significant bits each), which is
-// exact for a 24-bit significand; |mid| <= 2^-8 |x|, |lo| <= 2^-16 |x|. A product of two values is the six products of
-// parts down to 2^-16 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three left out are below 2^-23 of it
-// at worst and 2^-27 in the mean, of either sign. Each product of parts is exact in the MFMA's fp32, and the small
-// ones enter an accumulator first. Six bf16 MFMAs of k = 32 take 96 cycles where eight fp32 MFMAs of k = 4 take 256,
-// and a plane is read transposed, so a tensor is staged once instead of natural and transposed. Measured at B H = 64,
-// L = 400, D = 64 (fp32 MFMA -> split): forward 41.4 -> 31.9, backward 126 -> 85, bwd_bwd 328 -> 186 us, the error
-// against 64 bits 4.6e-7 -> 3.6e-7, 5.9e-7 -> 5.0e-7, 7.2e-7 -> 6.1e-7 (fewer roundings per sum).
-// Non-finite inputs (and values past bf16's range) do not survive the split: they give NaN wherever they enter; and parts
-// below bf16's normal range are taken as zero. A workgroup whose sums hold a NaN or a value below 2^-104 computes them
-// again with f32n (see redo_unsplit), so the results for such inputs are those of plain fp32 arithmetic.
+// Split products. 2^16 x = hi + mid + lo with each part the rest's rounding to bf16 (8 significant bits each), which is
+// exact for every finite fp32 x whose hi is finite, subnormal ones included: the last bit of x is worth 2^-149 or more,
+// that of a bf16 2^-133 (the bf16 MFMA and the conversion keep subnormals; without the scale the small parts of an
+// |x| < 2^-110 lost bits, 2^-9 of x itself near 2^-126). |mid| <= 2^-8 |hi|, |lo| <= 2^-16 |hi|. A product of two
+// values is the six products of parts down to 2^-16 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three left
+// out are below 2^-23 of it at worst and 2^-27 in the mean, of either sign. Each product of parts is exact in the MFMA's fp32,
+// and the small ones enter an accumulator first. Sums carry 2^32, which leaves at the end of a sum. Six bf16 MFMAs of
+// k = 32 take 96 cycles where eight fp32 MFMAs of k = 4 take 256, and a plane is read transposed, so a tensor is staged
+// once instead of natural and transposed. Measured at B H = 64, L = 400, D = 64 (fp32 MFMA -> split): forward
+// 45 -> 36, backward 126 -> 90, bwd_bwd 329 -> 190 us, the error against 64 bits 4.6e-7 -> 3.3e-7, 5.9e-7 -> 4.8e-7,
+// 7.2e-7 -> 5.9e-7 (fewer roundings per sum). A sum that is one product alone is less exact than on the fp32 MFMA: at
+// worst 9.9e-8 of it instead of 6.0e-8, 2.6e-8 instead of 2.5e-8 in the root mean square. The two products of 2^-24
+// (mid lo, lo mid) would close that and cost 10% (39, 96, 212 us); parts scaled by 2^8 and 2^16 of their own, with one
+// accumulator for each scale, cost 16% (39, 107, 221 us).
+// A non-finite input, or one past 2^111, does not survive the split: it gives NaN wherever it enters, and a sum past
+// 2^96 overflows. A workgroup with a sum that is not finite computes it again with f32n (see redo_unsplit), so the
+// results for such inputs are those of plain fp32 arithmetic.
 constexpr int NPLANE = 3;
+constexpr float PLANE_SCALE = 0x1p16f, PRODUCT_UNSCALE = 0x1p-32f;  // of a value's planes; off a product of two
 
 template <typename T> struct ET;
 
@@ -175,9 +183,11 @@ template <int DP> struct Lay<f32s, DP> {
     static constexpr int TRB = 0;
 };
 
-// Eight values as three planes of packed bf16.
+// Eight values as three planes of packed bf16 (scaled by PLANE_SCALE).
 __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u32x4 (&out)[NPLANE]) {
     float r[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] *= PLANE_SCALE;
 #pragma unroll
     for (int i = 0; i < NPLANE; ++i) {
         bf16x8 h;
@@ -190,14 +200,25 @@ __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u32x4 (&o
     }
 }
 
-// acc += sum over the six products of parts, the small ones first.
-__device__ __forceinline__ f32x4 mma_split(const u32x4 (&a)[NPLANE], const u32x4 (&b)[NPLANE], f32x4 acc) {
+// acc += the products of parts below hi hi, the small ones first.
+__device__ __forceinline__ f32x4 mma_split_small(const u32x4 (&a)[NPLANE], const u32x4 (&b)[NPLANE], f32x4 acc) {
     acc = ET<__bf16>::mma(a[2], b[0], acc);
     acc = ET<__bf16>::mma(a[0], b[2], acc);
     acc = ET<__bf16>::mma(a[1], b[1], acc);
     acc = ET<__bf16>::mma(a[1], b[0], acc);
-    acc = ET<__bf16>::mma(a[0], b[1], acc);
-    return ET<__bf16>::mma(a[0], b[0], acc);
+    return ET<__bf16>::mma(a[0], b[1], acc);
+}
+
+__device__ __forceinline__ f32x4 mma_split(const u32x4 (&a)[NPLANE], const u32x4 (&b)[NPLANE], f32x4 acc) {
+    return ET<__bf16>::mma(a[0], b[0], mma_split_small(a, b, acc));
+}
+
+// Takes the planes' scale out of the sums of a seq-contraction (mma_d takes it out itself).
+template <typename T, int N> __device__ __forceinline__ void unscale(f32x4 (&acc)[N]) {
+    if constexpr (ET<T>::SPLIT) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) acc[t] *= PRODUCT_UNSCALE;
+    }
 }
 
 // Column of chunk-local row x in the transposed LDS layout (see the header comment).
@@ -316,7 +337,7 @@ __device__ __forceinline__ float frag_dot(const OwnFrag<T, DP>& a, const OwnFrag
         if constexpr (ET<T>::SPLIT) {
             float x[8] = {}, y[8] = {};
 #pragma unroll
-            for (int i = NPLANE - 1; i >= 0; --i) {  // the parts' sum is the value
+            for (int i = NPLANE - 1; i >= 0; --i) {  // the parts' sum is the scaled value
                 const bf16x8 p = __builtin_bit_cast(bf16x8, a.v[c][i]), q = __builtin_bit_cast(bf16x8, b.v[c][i]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -338,26 +359,35 @@ __device__ __forceinline__ float frag_dot(const OwnFrag<T, DP>& a, const OwnFrag
             for (int e = 0; e < 8; ++e) s += (float)x[e] * (float)y[e];
         }
     }
-    return s;
+    return ET<T>::SPLIT ? s * PRODUCT_UNSCALE : s;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
 // d-contraction: acc[m = x][n = own] += sum_d Xn[x][d] * Own[own][d] for the 16 rows starting at Xn_tile.
+// SCORES: an overflow of the split sum becomes a NaN, so that it is seen (-inf would give P = 0); every other such sum is
+// multiplied into an accumulator as it is.
 // ---------------------------------------------------------------------------------------------------------------------
 
-template <typename T, int DP>
+template <typename T, int DP, bool SCORES = false>
 __device__ __forceinline__ void mma_d(f32x4& acc, const T* Xn_tile, const OwnFrag<T, DP>& f, int l16, int g) {
     using LY = Lay<T, DP>;
     if constexpr (ET<T>::SPLIT) {
         const unsigned char* base = reinterpret_cast<const unsigned char*>(Xn_tile);
+        u32x4 hi[LY::NC];
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < LY::NC; ++c) {
             u32x4 x[NPLANE];
 #pragma unroll
             for (int i = 0; i < NPLANE; ++i)
                 x[i] = *reinterpret_cast<const u32x4*>(base + i * LY::PLANE + Sw<DP>::off(l16, 4 * c + g));
-            acc = mma_split(x, f.v[c], acc);
+            hi[c] = x[0];
+            s = mma_split_small(x, f.v[c], s);
         }
+#pragma unroll
+        for (int c = 0; c < LY::NC; ++c) s = ET<__bf16>::mma(hi[c], f.v[c][0], s);
+        acc += s * PRODUCT_UNSCALE;
+        if constexpr (SCORES) acc += s * 0.f;
     } else {
         const T* p = Xn_tile + l16 * LY::PN + g * LY::VEC;
 #pragma unroll
@@ -553,7 +583,7 @@ template <typename T, int DP, int N> struct Stage {
 #pragma unroll
                 for (int t = 0; t < N; ++t) {
                     unsigned char* p = reinterpret_cast<unsigned char*>(Xn[t] ? Xn[t] : Xt[t]) + off;
-                    f32x4 e = __builtin_bit_cast(f32x4, r[t][i]);
+                    f32x4 e = __builtin_bit_cast(f32x4, r[t][i]) * PLANE_SCALE;
 #pragma unroll
                     for (int k = 0; k < NPLANE; ++k) {
                         bf16x4 h;

@@ -103,10 +103,10 @@ __device__ __forceinline__ void store_rows(void* out, int64_t row_off, const f32
 // Forward (row pass): online softmax over 32-key chunks.
 // =====================================================================================================================
 
-// Whether a lane's split sums hold a NaN, or a value so small that parts of its terms were subnormal (a bf16 MFMA takes
-// those as zero): below 2^-104, where the smallest parts, 2^-16 of theirs, come within 2^6 of the smallest normal, 2^-126.
+// Whether a lane's split sums hold a NaN or an infinity. Nothing else needs a second look: the split is exact for every
+// finite operand that its scale does not push past bf16's range, and one past it makes every sum it enters a NaN.
 template <typename T> __device__ __forceinline__ bool unsplit(float v) {
-    return ET<T>::SPLIT && !(fabsf(v) >= 0x1p-104f || v == 0.f);
+    return ET<T>::SPLIT && !(fabsf(v) <= FLT_MAX);
 }
 template <typename T, int N> __device__ __forceinline__ bool unsplit(const f32x4 (&v)[N]) {
     bool any = false;
@@ -120,8 +120,9 @@ template <typename T, int N> __device__ __forceinline__ bool unsplit(const f32x4
 }
 
 // Runs ``body`` (which returns whether a sum of this lane is one of those) with T; split products give NaN for
-// non-finite inputs where fp32 arithmetic may give an infinity, and lose bits of values near 2^-126, so a workgroup that
-// saw either runs again with f32n, which overwrites everything the first run wrote.
+// non-finite inputs where fp32 arithmetic may give an infinity, and overflow earlier, so a workgroup that saw either
+// runs again with f32n, which overwrites everything the first run wrote (both runs, with a NaN in every workgroup, at 64
+// slices, L = 400, D = 64: 71, 203, 468 us where the split alone takes 36, 90, 190).
 template <typename T, class Body> __device__ __forceinline__ void redo_unsplit(Body&& body) {
     const bool bad = body(T{});
     if constexpr (ET<T>::SPLIT) {
@@ -178,8 +179,8 @@ template <typename T, int DP> __device__ __forceinline__ bool fwd_pass(const Arg
         const T* Kn = reinterpret_cast<const T*>(smem + buf * FS::ONE);
         const T* Vt = reinterpret_cast<const T*>(smem + buf * FS::ONE + LY::NATB);
         f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-        mma_d<T, DP>(s0, Kn, qf, w.l16, w.g);
-        mma_d<T, DP>(s1, Kn + 16 * LY::PN, qf, w.l16, w.g);
+        mma_d<T, DP, true>(s0, Kn, qf, w.l16, w.g);
+        mma_d<T, DP, true>(s1, Kn + 16 * LY::PN, qf, w.l16, w.g);
         float mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -228,6 +229,7 @@ template <typename T, int DP> __device__ __forceinline__ bool fwd_pass(const Arg
     }
     if (!active) return false;
     lsum = xsum4(lsum);
+    unscale<T>(acc);
     const bool redo = unsplit<T>(acc) || unsplit<T>(lsum);
     if (own < L) {
         const int64_t r = (int64_t)bh * L + own;
@@ -310,8 +312,8 @@ template <typename T, int DP, bool FUSED> struct BwdRow {
         const int L = a.L;
         const float sc = a.scale;
         f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, d0 = p0, d1 = p0;
-        mma_d<T, DP>(p0, Kn, qf, w.l16, w.g);
-        mma_d<T, DP>(p1, Kn + 16 * LY::PN, qf, w.l16, w.g);
+        mma_d<T, DP, true>(p0, Kn, qf, w.l16, w.g);
+        mma_d<T, DP, true>(p1, Kn + 16 * LY::PN, qf, w.l16, w.g);
         mma_d<T, DP>(d0, Vn, df, w.l16, w.g);
         mma_d<T, DP>(d1, Vn + 16 * LY::PN, df, w.l16, w.g);
 #pragma unroll
@@ -328,6 +330,7 @@ template <typename T, int DP, bool FUSED> struct BwdRow {
     }
     __device__ __forceinline__ bool redo(int L) const { return active && own < L && unsplit<T>(acc); }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
+        unscale<T>(acc);
         if (active && own < a.L) store_rows<T, DP>(a.out0, ((int64_t)bh * a.L + own) * a.D, acc, a.scale, a.D, w.g);
     }
 };
@@ -375,8 +378,8 @@ template <typename T, int DP> struct BwdCol {
         const f32x4 r0 = *reinterpret_cast<const f32x4*>(st + ss + 4 * w.g);
         const f32x4 r1 = *reinterpret_cast<const f32x4*>(st + ss + 16 + 4 * w.g);
         f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, d0 = p0, d1 = p0;
-        mma_d<T, DP>(p0, Qn, kf, w.l16, w.g);
-        mma_d<T, DP>(p1, Qn + 16 * LY::PN, kf, w.l16, w.g);
+        mma_d<T, DP, true>(p0, Qn, kf, w.l16, w.g);
+        mma_d<T, DP, true>(p1, Qn + 16 * LY::PN, kf, w.l16, w.g);
         mma_d<T, DP>(d0, On, vf, w.l16, w.g);
         mma_d<T, DP>(d1, On + 16 * LY::PN, vf, w.l16, w.g);
 #pragma unroll
@@ -398,6 +401,8 @@ template <typename T, int DP> struct BwdCol {
         return active && own < L && (unsplit<T>(ak) || unsplit<T>(av));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
+        unscale<T>(ak);
+        unscale<T>(av);
         if (active && own < a.L) {
             const int64_t r = ((int64_t)bh * a.L + own) * a.D;
             store_rows<T, DP>(a.out1, r, ak, a.scale, a.D, w.g);
@@ -471,7 +476,7 @@ template <typename T, int DP, bool FUSED> struct BbRow {
         for (int hh = 0; hh < 2; ++hh) {
             p[hh] = dp[hh] = at[hh] = bm[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
             const int off = hh * 16 * LY::PN;
-            mma_d<T, DP>(p[hh], Kn + off, qf, w.l16, w.g);
+            mma_d<T, DP, true>(p[hh], Kn + off, qf, w.l16, w.g);
             mma_d<T, DP>(at[hh], Kn + off, gqf, w.l16, w.g);
             mma_d<T, DP>(at[hh], gKn + off, qf, w.l16, w.g);
             mma_d<T, DP>(dp[hh], Vn + off, df, w.l16, w.g);
@@ -538,6 +543,10 @@ template <typename T, int DP, bool FUSED> struct BbRow {
                (unsplit<T>(X) || unsplit<T>(U) || unsplit<T>(Z) || unsplit<T>(Wv) || unsplit<T>(e_acc + t_acc));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w, float* st) {
+        unscale<T>(X);
+        unscale<T>(U);
+        unscale<T>(Z);
+        unscale<T>(Wv);
         const float E = xsum4(e_acc);
         const float Tm = xsum4(t_acc);
         const int L = a.L, D = a.D;
@@ -620,7 +629,7 @@ template <typename T, int DP> struct BbCol {
         for (int hh = 0; hh < 2; ++hh) {
             p[hh] = dp[hh] = at[hh] = bm[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
             const int off = hh * 16 * LY::PN;
-            mma_d<T, DP>(p[hh], Qn + off, kf, w.l16, w.g);
+            mma_d<T, DP, true>(p[hh], Qn + off, kf, w.l16, w.g);
             mma_d<T, DP>(at[hh], Qn + off, gkf, w.l16, w.g);
             mma_d<T, DP>(at[hh], gQn + off, kf, w.l16, w.g);
             mma_d<T, DP>(dp[hh], On + off, vf, w.l16, w.g);
@@ -659,6 +668,8 @@ template <typename T, int DP> struct BbCol {
         return active && own < L && (unsplit<T>(hk) || unsplit<T>(hv));
     }
     __device__ __forceinline__ void finish(const Args& a, const WaveIds& w) {
+        unscale<T>(hk);
+        unscale<T>(hv);
         if (active && own < a.L) {
             const int64_t r = ((int64_t)bh * a.L + own) * a.D;
             store_rows<T, DP>(a.out1, r, hk, a.scale, a.D, w.g);
@@ -986,8 +997,8 @@ static int persistent_grid(const void* kernel, int threads, int64_t work) {
 template <typename T> constexpr bool one_workgroup(int dp) { return dp <= (ET<T>::SPLIT ? 32 : 128); }
 
 // fp32 as split products (f32s): every L > 128, and D in 17..32 from L = 33 on. Against the fp32 MFMA, forward /
-// backward / bwd_bwd in us: 64 slices, L = 400, D = 64: 31.6 / 85 / 185 against 41 / 126 / 328; 8 slices, L = 300,
-// D = 128: 28 / 89 / 196 against 38 / 116 / 287; 512 slices, L = 100, D = 32: 13 / 31 / 69 against 16 / 40 / 102. Below
+// backward / bwd_bwd in us: 64 slices, L = 400, D = 64: 36 / 90 / 190 against 45 / 126 / 329; 8 slices, L = 300,
+// D = 128: 31 / 84 / 209 against 38 / 116 / 287; 512 slices, L = 100, D = 32: 15 / 35 / 77 against 17 / 43 / 103. Below
 // those lines it loses: a wave that runs both passes of bwd_bwd spills from D = 64 on (50 against 37 at 256 slices,
 // L = 64, D = 64; 474 against 309 at 128 slices, L = 100, D = 128), and one chunk is mostly its own split and stores
 // (2,048 slices, L = 30, D = 128: 42 / 141 / 716 against 29 / 112 / 618). The three ops of a shape take the same side,

@@ -1,6 +1,8 @@
 """fp32 attention as split products (three bf16 planes per value): parity at the edges of its range, precision against
 the fp64 oracle, and non-finite and huge inputs, which it hands to the fp32 MFMA."""
 
+import math
+
 import pytest
 import torch
 
@@ -90,6 +92,56 @@ def test_tiny_values_keep_their_precision(shape, size):
     dv = ops._hip_bwd(q, k, v, o, lse, do * size, scale)[2].cpu().double()
     want = p.transpose(-1, -2) @ (do * size).cpu().double()
     assert ((dv - want).norm() / want.norm()).item() < 1.5e-6
+
+
+SCALED = {  # powers of two on q, k, v, dO, gQ, gK, gV that leave the probabilities as they are
+    "small dO against large k": (-20, 20, 0, -118, -20, 20, 0),
+    "small q against large k": (-118, 118, 0, 0, -118, 118, 0),
+    "small v against large dO": (0, 0, -118, 118, 0, 0, -118),
+    "small cotangents": (0, 0, 0, 0, -118, -118, -118),
+}
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 140, 64), (1, 1, 50, 32), (1, 1, 130, 128)])
+@pytest.mark.parametrize("powers", SCALED.values(), ids=SCALED.keys())
+def test_every_output_keeps_its_precision_on_scaled_operands(shape, powers):
+    """Operands near 2^-126 (a plane of unscaled remainders would lose their low bits) beside ones that make up for it:
+    the sums and the outputs are ordinary numbers, so their size says nothing about the operands."""
+    B, H, L, D = shape
+    ts = oracle.make_inputs(B, H, L, D, dtype=F32, seed=3, qkv_scale=0.7)
+    ts = [t * 2.0**p for t, p in zip(ts, powers)]
+    scale = D**-0.5
+    got = _run(*(t.cuda() for t in ts), scale)
+    q, k, v, do, gq, gk, gv = (t.double() for t in ts)
+    o, lse = oracle.attn_fwd(q, k, v, scale)
+    want = [o, lse, *oracle.attn_bwd(q, k, v, o, lse, do, scale),
+            *oracle.attn_bwd_bwd(q, k, v, o, lse, do, None, gq, gk, gv, scale)]
+    for name, a, r in zip(("o", "lse", "dq", "dk", "dv", "hq", "hk", "hv", "hdo"), got, want):
+        # as on ordinary operands, plus, where an output is subnormal, half a quantum for each of its sums' L terms
+        bound = 1.5e-6 * r.norm() + L * 2.0**-150 * r.numel() ** 0.5
+        assert (a.double().cpu() - r).norm() <= bound, name
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 140, 64), (1, 1, 50, 32)])
+def test_scores_that_overflow_only_before_the_scale(shape):
+    """Sums of q k around -2^96, where the planes' own scale overflows some of a row's, with a scale that makes ordinary
+    scores of them."""
+    B, H, L, D = shape
+    q, k, v, do, gq, gk, gv = oracle.make_inputs(B, H, L, D, dtype=F32, seed=5, qkv_scale=0.7)
+    q, k = q.abs(), -k.abs()
+    q = q * -(2.0**48 / (q @ k.transpose(-1, -2)).mean(-1, keepdim=True))  # a row's scores lie around -2^48 of k's unit
+    k, gq, gk = k * 2.0**48, gq * 2.0**48, gk * 2.0**48
+    ts, scale = (q, k, v, do, gq, gk, gv), 2.0**-92
+    s = q.double() @ k.double().transpose(-1, -2)
+    assert (s < -(2.0**96)).any(-1).all() and (s > -(2.0**96)).any(-1).all()  # every row has scores on either side
+    got = _run(*(t.cuda() for t in ts), scale)
+    q, k, v, do, gq, gk, gv = (t.double() for t in ts)
+    o, lse = oracle.attn_fwd(q, k, v, scale)
+    want = [o, lse, *oracle.attn_bwd(q, k, v, o, lse, do, scale),
+            *oracle.attn_bwd_bwd(q, k, v, o, lse, do, None, gq, gk, gv, scale)]
+    # scores of about -16, each rounded to 2^-24 of itself before the exponential
+    for name, a, r in zip(("o", "lse", "dq", "dk", "dv", "hq", "hk", "hv", "hdo"), got, want):
+        assert (a.double().cpu() - r).norm() <= 16 * 2.0**-22 * r.norm(), name
 
 
 def test_repeated_calls_give_the_same_bits():
