@@ -339,21 +339,21 @@ template <typename T, int S, int VW> __global__ __launch_bounds__(256) void k_sp
 #pragma clang fp contract(off)
     using F = float __attribute__((ext_vector_type(VW)));
     using V = T __attribute__((ext_vector_type(VW)));
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VW;
-    if (i >= n) return;
-    F v[S];
+    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VW; i < n; i += (int64_t)gridDim.x * 256 * VW) {
+        F v[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const F*>(part + s * n + i);
+        for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const F*>(part + s * n + i);
 #pragma unroll
-    for (int w = S / 2; w >= 1; w >>= 1)
+        for (int w = S / 2; w >= 1; w >>= 1)
 #pragma unroll
-        for (int s = 0; s < w; ++s)
+            for (int s = 0; s < w; ++s)
 #pragma unroll
-            for (int e = 0; e < VW; ++e) v[s][e] += v[s + w][e];
-    V o;
+                for (int e = 0; e < VW; ++e) v[s][e] += v[s + w][e];
+        V o;
 #pragma unroll
-    for (int e = 0; e < VW; ++e) o[e] = (T)v[0][e];
-    *reinterpret_cast<V*>(out + i) = o;
+        for (int e = 0; e < VW; ++e) o[e] = (T)v[0][e];
+        *reinterpret_cast<V*>(out + i) = o;
+    }
 }
 
 static int rc_launch() {
@@ -408,14 +408,15 @@ template <int MODE> static void launch_norm(int dtype, hipStream_t s, const Norm
 // 5.3 TB/s at [64000, 2 x 1536] bf16 (forward 110, backward 183 us), one vector each at 5.8 (102, 171). Non-temporal
 // stores made the backward alone faster (84 -> 73 us at 31,104 rows) and a block slower (2,720 -> 2,728 us): the next
 // product reads the rows from the last-level cache.
-constexpr int64_t GLU_MAX_BLOCKS = (int64_t)1 << 24;
+constexpr int64_t MAX_BLOCKS = ((int64_t)1 << 24) - 1;  // of 256 threads
+static_assert(MAX_BLOCKS * 256 < ((int64_t)1 << 32), "a launch holds fewer than 2^32 threads in a dimension");
 
 template <typename T, int MODE> static void launch_glu_t(hipStream_t s, const GluArgs& a, bool vec_ok) {
     constexpr int VEC = 16 / (int)sizeof(T);
     if (vec_ok && a.I % VEC == 0) {
         const int64_t total = a.n * (a.I / VEC);
         const int64_t want = (total + 255) / 256;
-        const dim3 grid((unsigned)(want < GLU_MAX_BLOCKS ? want : GLU_MAX_BLOCKS)), block(256);
+        const dim3 grid((unsigned)(want < MAX_BLOCKS ? want : MAX_BLOCKS)), block(256);
         // 32-bit indices when every element offset (2 I per row) fits
         if (a.n * 2 * (int64_t)a.I < ((int64_t)1 << 31)) hipLaunchKernelGGL((k_swiglu_vec<T, MODE, uint32_t>), grid, block, 0, s, a);
         else hipLaunchKernelGGL((k_swiglu_vec<T, MODE, int64_t>), grid, block, 0, s, a);
@@ -437,8 +438,8 @@ template <int MODE> static void launch_glu(int dtype, hipStream_t s, const GluAr
 
 template <typename T, int S> static void launch_split_sum(hipStream_t st, const float* part, int64_t n, T* out) {
     const bool vec = n % 4 == 0 && aligned16(part) && ((uintptr_t)out & 7) == 0;
-    const int64_t per = 256 * (vec ? 4 : 1);
-    const dim3 grid((unsigned)((n + per - 1) / per)), block(256);
+    const int64_t per = 256 * (vec ? 4 : 1), want = (n + per - 1) / per;
+    const dim3 grid((unsigned)(want < MAX_BLOCKS ? want : MAX_BLOCKS)), block(256);
     if (vec) hipLaunchKernelGGL((k_split_sum<T, S, 4>), grid, block, 0, st, part, n, out);
     else hipLaunchKernelGGL((k_split_sum<T, S, 1>), grid, block, 0, st, part, n, out);
 }

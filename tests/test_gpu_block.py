@@ -12,7 +12,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from ebr_amd import block
+from ebr_amd import _capi, block
 from ebr_amd import energy as en
 from ebr_amd import layers
 
@@ -165,3 +165,23 @@ def test_ops_reject_mismatched_operands_and_take_empty_inputs(cuda):
     xe = e.clone().requires_grad_(True)
     (dx,) = torch.autograd.grad(block.rms_norm(xe, EPS).sum(), xe, create_graph=True)
     assert dx.shape == (0, 64)
+
+
+def test_split_sum_past_one_grid():
+    """More elements than a launch holds threads: every one is summed (2^32 + 5, an odd count, one element per thread)."""
+    n = 2**32 + 5
+    if torch.cuda.mem_get_info()[0] < 60 * 2**30:
+        pytest.skip("needs 43 GB")
+    part = torch.ones((2, n), device="cuda")
+    marks = [0, 1, 2**32 - 257, 2**32 - 256, 2**32 - 1, 2**32, n - 1]
+    for i in marks:
+        part[1, i] = 2.0
+    out = torch.zeros((n,), device="cuda", dtype=torch.bfloat16)
+    rc = _capi.load().ebr_block_split_sum(_capi.DTYPE_BF16, 2, n, part.data_ptr(), out.data_ptr(), None)
+    torch.cuda.synchronize()
+    assert rc == 0
+    assert out[marks].eq(3.0).all()
+    out[marks] = 2.0
+    del part
+    lo, hi = out.aminmax()
+    assert lo.item() == hi.item() == 2.0
