@@ -1244,7 +1244,8 @@ template <typename T, int DP> struct BbLaunch {
             if (a.plan == EBR_PLAN_LONG) return EBR_ERR_PLAN;
             if (a.plan == EBR_PLAN_GENERIC || !resident_shape(a, DP, (int)sizeof(T), true)) {
                 if (!plan_allows(a, EBR_PLAN_GENERIC)) return EBR_ERR_PLAN;
-                if constexpr (one_workgroup<T>(DP)) hipLaunchKernelGGL((k_bb_fused<T, DP>), grid, block, 0, s, a);
+                if constexpr (!one_workgroup<T>(DP)) return EBR_ERR_PLAN;  // dispatch sends none of these here
+                else hipLaunchKernelGGL((k_bb_fused<T, DP>), grid, block, 0, s, a);
             } else if constexpr (!ET<T>::WIDE) {
                 const int nch = (a.L + CH - 1) / CH;
                 // tiles shared through LDS, persistent with loader waves (k_bb_share), where its regions fit the LDS:
