@@ -332,8 +332,9 @@ template <typename T, int MODE, typename IDX> __global__ __launch_bounds__(256) 
 
 // out[i] = round(sum over s of part[s][i]) of S fp32 partial products [S, n]: the sum and the narrowing of a split-K
 // weight gradient, which as two ops wrote the fp32 sum and read it again. HBM-bound; a thread has all S loads of its
-// vector in flight and adds them pairwise. bf16: S = 8, n = 3072 x 512, 17.5 us as two ops, 9.9 here (5.4 TB/s); S = 16,
-// n = 1536 x 512, 16 and 7.5 us (6.9 TB/s, the partials still in the last-level cache).
+// vector in flight. They are added in the order of those two ops (four interleaved sums, then these in turn), so that
+// the gradient has the same bits on either path. bf16: S = 8, n = 3072 x 512, 17.5 us as two ops, 9.9 here (5.4 TB/s);
+// S = 16, n = 1536 x 512, 16 and 7.5 us (6.9 TB/s, the partials still in the last-level cache).
 template <typename T, int S, int VW> __global__ __launch_bounds__(256) void k_split_sum(const float* part, int64_t n,
                                                                                          T* out) {
 #pragma clang fp contract(off)
@@ -344,11 +345,13 @@ template <typename T, int S, int VW> __global__ __launch_bounds__(256) void k_sp
 #pragma unroll
         for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const F*>(part + s * n + i);
 #pragma unroll
-        for (int w = S / 2; w >= 1; w >>= 1)
+        for (int s = 4; s < S; ++s)
 #pragma unroll
-            for (int s = 0; s < w; ++s)
+            for (int e = 0; e < VW; ++e) v[s & 3][e] += v[s][e];
 #pragma unroll
-                for (int e = 0; e < VW; ++e) v[s][e] += v[s + w][e];
+        for (int s = 1; s < (S < 4 ? S : 4); ++s)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) v[0][e] += v[s][e];
         V o;
 #pragma unroll
         for (int e = 0; e < VW; ++e) o[e] = (T)v[0][e];

@@ -127,6 +127,7 @@ def test_split_weight_gradients(dtype, rows, N, K):
     # fp32 sums of exact products, rounded once: half an ulp of the dtype, plus the sums' own error
     eps = torch.finfo(dtype).eps
     assert ((got.double() - want).abs() <= 0.51 * eps * want.abs() + 1e-5 * rows**0.5).all()
+    assert torch.equal(got, linear.weight_grad(dy, x))  # the partials' sum and its rounding as ops of their own
 
 
 @gpu
