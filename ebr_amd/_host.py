@@ -4,6 +4,10 @@ launches of the GPU ops without Python in between.
 ``module()`` is the loaded extension, or None when it is not there or does not load with this torch: the Python layer
 then runs the same kernels of ``libebr_attn.so`` (and raises if that is missing). Each of its functions returns None for
 a call that the Python layer has to take (see the source's header); callers go on in Python then.
+
+``GRADS``: the Python formulas of the native nodes' gradients, by node. A native node whose backward runs under a
+transform (``is_grads_batched``), a mode or a hook, or with cotangents that are no plain tensors, calls its formula: the
+saved values, then the cotangents (None where there is none), and gets the inputs' gradients.
 """
 
 from __future__ import annotations
@@ -12,6 +16,7 @@ import importlib.machinery
 import importlib.util
 import threading
 import warnings
+from typing import Callable, Dict
 
 import torch  # noqa: F401  (the extension links against torch's libraries)
 
@@ -19,6 +24,19 @@ from ebr_amd import _capi
 
 NAME = "ebr_host"
 PATH = _capi.LIB_PATH.with_name(NAME + ".so")
+
+GRADS: Dict[str, Callable] = {}
+
+
+def gradient(node: str) -> Callable[[Callable], Callable]:
+    """Registers the decorated function as a native node's Python gradient."""
+
+    def register(fn: Callable) -> Callable:
+        GRADS[node] = fn
+        return fn
+
+    return register
+
 
 _LOCK = threading.Lock()
 _TRIED = False
@@ -49,4 +67,4 @@ def module():
     return _MODULE if _TRIED else _load()
 
 
-__all__ = ["module"]
+__all__ = ["GRADS", "gradient", "module"]

@@ -161,6 +161,17 @@ class _RmsNorm(torch.autograd.Function):
         return _RmsNormBwd.apply(x, dy, ctx.eps), None
 
 
+@_host.gradient("rms_norm")
+def _rms_norm_grads(x, eps, dy, acc):
+    dx = _RmsNormBwd.apply(x, dy, eps)
+    return (dx if acc is None else dx + acc,)
+
+
+@_host.gradient("rms_norm_bwd")
+def _rms_norm_bwd_grads(x, dy, eps, c):
+    return torch.ops.ebr_fused.block_rmsnorm_bwd2(x, dy, c, eps)
+
+
 # ---------------------------------------------------------------------------------------------------------------------
 # SwiGLU
 # ---------------------------------------------------------------------------------------------------------------------
@@ -262,6 +273,17 @@ class _SwiGLU(torch.autograd.Function):
     def backward(ctx, dy):
         (gu,) = ctx.saved_tensors
         return _SwiGLUBwd.apply(gu, dy)
+
+
+@_host.gradient("swiglu")
+def _swiglu_grads(gu, dy, acc):
+    dgu = _SwiGLUBwd.apply(gu, dy)
+    return (dgu if acc is None else dgu + acc,)
+
+
+@_host.gradient("swiglu_bwd")
+def _swiglu_bwd_grads(gu, dy, c):
+    return torch.ops.ebr_fused.block_swiglu_bwd2(gu, dy, c)
 
 
 def rms_norm(x: Tensor, eps: float) -> Tensor:

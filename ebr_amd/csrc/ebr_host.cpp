@@ -5,7 +5,9 @@
 // fakes and their autograd Functions, and stays the path of every call this file does not take: tensor subclasses and
 // fake tensors, torch.func transforms, dispatch and function modes, tracing, forward-mode duals, saved-tensor hooks,
 // tensors off the GPU, and every argument the Python layer would refuse or pad. Each entry point below returns None for
-// those, and the caller goes on in Python.
+// those, and the caller goes on in Python. A node asks again when it runs: a backward under a transform (batched
+// gradients), a mode, a tracer or hooks, or with cotangents of another kind, takes the Python formulas of its gradient
+// (python_grads).
 //
 // Why it exists: a graded attention step (three launches) spent 453 us on the host in Python (autograd Functions,
 // custom-op dispatch, ctypes marshalling, GIL hand-overs to the engine's threads) against 45 us of kernel time for one
@@ -55,16 +57,45 @@ bool plain_context() {
            !torch::jit::tracer::isTracing() && !at::SavedTensorDefaultHooks::get_hooks().has_value();
 }
 
-// The tensor behind a Python argument if it is an ordinary dense GPU tensor, else an undefined one.
+// An ordinary dense GPU tensor.
+bool plain_tensor(const Tensor& t) {
+    static const c10::DispatchKeySet allowed({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
+                                              c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
+    return t.defined() && t.is_cuda() && (t.key_set().raw_repr() & ~allowed.raw_repr()) == 0 && !t.is_inference() &&
+           !t._fw_grad(/*level=*/0).defined();
+}
+
+// The tensor behind a Python argument if it is one of those, else an undefined one.
 Tensor plain(const py::handle& h) {
     if (!THPVariable_CheckExact(h.ptr())) return {};
     const Tensor& t = THPVariable_Unpack(h.ptr());
-    static const c10::DispatchKeySet allowed({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
-                                              c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
-    if (!t.defined() || !t.is_cuda() || (t.key_set().raw_repr() & ~allowed.raw_repr()) != 0 || t.is_inference())
-        return {};
-    if (t._fw_grad(/*level=*/0).defined()) return {};
-    return t;
+    return plain_tensor(t) ? t : Tensor();
+}
+
+// Whether a node's backward runs here: its saved tensors were plain when it was made, its cotangents and the context have
+// to be now.
+bool native(const variable_list& grads) {
+    for (const Tensor& t : grads)
+        if (t.defined() && !plain_tensor(t)) return false;
+    return plain_context();
+}
+
+// A node's gradients by its Python formula (ebr_amd._host.GRADS), which runs the ops through the dispatcher.
+template <class... Args> variable_list python_grads(const char* name, size_t n, const Args&... args) {
+    const py::gil_scoped_acquire gil;
+    try {
+        const py::tuple r = py::module_::import("ebr_amd._host").attr("GRADS")[name](args...);
+        TORCH_CHECK(r.size() <= n, name, ": ", r.size(), " gradients for ", n, " inputs");
+        variable_list out(n);
+        for (size_t i = 0; i < r.size(); ++i)
+            if (!r[i].is_none()) out[i] = r[i].cast<Tensor>();
+        return out;
+    } catch (py::error_already_set& e) {
+        e.restore();
+        python_error err;
+        err.persist();
+        throw err;
+    }
 }
 
 int dtype_code(at::ScalarType t) {
@@ -229,6 +260,8 @@ struct AttnBwd : Function<AttnBwd> {
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         const variable_list s = ctx->get_saved_variables();
         const double scale = ctx->saved_data["scale"].toDouble();
+        if (!native(g))
+            return python_grads("attention_bwd", 7, s[0], s[1], s[2], s[3], s[4], s[5], scale, g[0], g[1], g[2]);
         Tensor cot[3];
         for (int i = 0; i < 3; ++i)
             cot[i] = g[i].defined() ? g[i] : at::zeros({s[i].size(3)}, s[i].options()).expand(s[i].sizes());
@@ -253,7 +286,9 @@ struct AttnFwd : Function<AttnFwd> {
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return variable_list(4);  // only AttnBwd used o: nothing to add
         const variable_list s = ctx->get_saved_variables();
-        variable_list d = AttnBwd::apply(s[0], s[1], s[2], s[3], s[4], g[0], ctx->saved_data["scale"].toDouble());
+        const double scale = ctx->saved_data["scale"].toDouble();
+        if (!native(g)) return python_grads("attention", 4, s[0], s[1], s[2], s[3], s[4], scale, g[0]);
+        variable_list d = AttnBwd::apply(s[0], s[1], s[2], s[3], s[4], g[0], scale);
         d.emplace_back();
         return d;
     }
@@ -334,7 +369,9 @@ struct RopeMerge : Function<RopeMerge> {
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return variable_list(6);
         const variable_list s = ctx->get_saved_variables();
-        variable_list d = RopeSplit::apply(g[0], s[0], s[1], maybe(s[2]), ctx->saved_data["heads"].toInt());
+        const int64_t heads = ctx->saved_data["heads"].toInt();
+        if (!native(g)) return python_grads("rope_merge", 6, s[0], s[1], s[2], heads, g[0]);
+        variable_list d = RopeSplit::apply(g[0], s[0], s[1], maybe(s[2]), heads);
         d.resize(6);
         return d;
     }
@@ -347,9 +384,10 @@ variable_list RopeSplit::backward(AutogradContext* ctx, const variable_list& g) 
     for (const Tensor& t : g)
         if (t.defined()) some = t;
     if (!some.defined()) return out;
+    const variable_list s = ctx->get_saved_variables();
+    if (!native(g)) return python_grads("rope_split", 5, s[0], s[1], s[2], shape, g[0], g[1], g[2]);
     Tensor d[3];
     for (int i = 0; i < 3; ++i) d[i] = g[i].defined() ? g[i] : at::zeros({shape[3]}, some.options()).expand(shape);
-    const variable_list s = ctx->get_saved_variables();
     out[0] = RopeMerge::apply(d[0], d[1], d[2], s[0], s[1], maybe(s[2]))[0];
     return out;
 }
@@ -466,6 +504,9 @@ struct RopeAttnBwd : Function<RopeAttnBwd> {
         const variable_list s = ctx->get_saved_variables();
         const Tensor &t = s[0], &q = s[1], &dy = s[4];
         const int64_t heads = q.size(1);
+        if (!native(g))
+            return python_grads("rope_attention_bwd", 10, t, q, s[2], s[3], dy, s[5], s[6], s[7], s[8], s[9],
+                                ctx->saved_data["scale"].toDouble(), want_t, g[0]);
         const variable_list c = split_graded(g[0].to(q.scalar_type()), s[7], s[8], t, want_t ? s[9] : Tensor(), heads);
         const variable_list h = attn_bwd_bwd(q, s[2], s[3], s[5], s[6], heads_apart(dy, heads), c[0], c[1], c[2],
                                              ctx->saved_data["scale"].toDouble());
@@ -496,6 +537,9 @@ struct RopeAttn : Function<RopeAttn> {
         const Tensor &qkv = s[0], &t = s[1], &cos = s[2], &sin = s[3], &q = s[4], &k = s[5], &v = s[6];
         const int64_t heads = q.size(1);
         const double scale = ctx->saved_data["scale"].toDouble();
+        if (!native(g))
+            return python_grads("rope_attention", 6, qkv, t, cos, sin, q, k, v, s[7], s[8], scale, want_t, dy, g[1],
+                                g[2], g[3]);
         if (at::GradMode::is_enabled()) {
             if (!more && !want_t) {
                 out[0] = RopeAttnBwd::apply(t, q, k, v, dy, s[7], s[8], cos, sin, scale)[0];
@@ -638,6 +682,7 @@ struct RmsNormBwd : Function<RmsNormBwd> {
         if (!g[0].defined()) return variable_list(3);
         const variable_list s = ctx->get_saved_variables();
         const double eps = ctx->saved_data["eps"].toDouble();
+        if (!native(g)) return python_grads("rms_norm_bwd", 3, s[0], s[1], eps, g[0]);
         variable_list d = rmsnorm_bwd2(s[0], s[1], g[0], eps);
         if (recorded({s[0], s[1], g[0]})) d = last(std::move(d));
         d.emplace_back();
@@ -652,6 +697,7 @@ Tensor own_input(const Tensor& x) { return x.detach(); }
 // The gradient of a norm's input: from dy through the backward's node, plus ``acc``.
 Tensor norm_grad(const Tensor& x, const Tensor& dy, const Tensor& acc, double eps) {
     if (!dy.defined()) return acc;
+    if (!native({dy, acc})) return python_grads("rms_norm", 1, x, eps, dy, acc)[0];
     if (acc.defined() && !at::GradMode::is_enabled()) return rmsnorm_bwd(x, dy, acc, eps);
     const Tensor dx = RmsNormBwd::apply(x, dy, eps)[0];
     return acc.defined() ? dx + acc : dx;
@@ -741,6 +787,7 @@ struct SwiGLUBwd : Function<SwiGLUBwd> {
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return variable_list(2);
         const variable_list s = ctx->get_saved_variables();
+        if (!native(g)) return python_grads("swiglu_bwd", 2, s[0], s[1], g[0]);
         variable_list d = swiglu_bwd2(s[0], s[1], g[0]);
         return recorded({s[0], s[1], g[0]}) ? last(std::move(d)) : d;
     }
@@ -756,6 +803,7 @@ struct SwiGLU : Function<SwiGLU> {
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
         if (!g[0].defined()) return {g[1]};
         const Tensor gu = ctx->get_saved_variables()[0];
+        if (!native(g)) return python_grads("swiglu", 1, gu, g[0], g[1]);
         if (g[1].defined() && !at::GradMode::is_enabled()) return {swiglu_bwd(gu, g[0], g[1])};
         const Tensor d = SwiGLUBwd::apply(gu, g[0])[0];
         return {g[1].defined() ? d + g[1] : d};
@@ -838,6 +886,7 @@ struct NoisyPoint : Function<NoisyPoint> {
         if (!g[0].defined()) return out;
         const Tensor z = ctx->get_saved_variables()[0];
         const double eps = ctx->saved_data["eps"].toDouble();
+        if (!native(g)) return python_grads("noisy_point", 4, z, eps, g[0]);
         out[0] = noisy_bwd(z, g[0], eps);
         if (recorded({z, g[0]})) out[0] = last({out[0]})[0];
         return out;
@@ -869,6 +918,7 @@ struct StepProject : Function<StepProject> {
         if (!gr[0].defined()) return out;
         const variable_list s = ctx->get_saved_variables();
         const double eps = ctx->saved_data["eps"].toDouble();
+        if (!native(gr)) return python_grads("step_project", 6, s[0], s[1], s[2], s[3], s[4], eps, gr[0]);
         variable_list d = step_bwd(s[0], s[1], s[2], s[3], s[4], gr[0], eps);
         if (recorded({s[0], s[1], gr[0]})) d = last(std::move(d));
         out[0] = d[0];
@@ -992,6 +1042,7 @@ struct Linear : Function<Linear> {  // Y = X W^T
         if (!g[0].defined()) return out;
         const bool nx = ctx->needs_input_grad(0), nw = ctx->needs_input_grad(1);
         const variable_list s = ctx->get_saved_variables();
+        if (!native(g)) return python_grads("linear", 2, s[0], s[1], g[0], nx, nw);
         if (nx) out[0] = Dgrad::apply(g[0], s[1])[0];
         if (nw) out[1] = weight_grad(g[0], s[0]);
         return out;
@@ -1003,6 +1054,7 @@ variable_list Dgrad::backward(AutogradContext* ctx, const variable_list& g) {
     if (!g[0].defined()) return out;
     const bool ndy = ctx->needs_input_grad(0), nw = ctx->needs_input_grad(1);
     const variable_list s = ctx->get_saved_variables();
+    if (!native(g)) return python_grads("linear_dgrad", 2, s[0], s[1], g[0], ndy, nw);
     if (ndy) out[0] = at::GradMode::is_enabled() ? Linear::apply(g[0], s[1])[0] : at::linear(g[0], s[1]);
     if (nw) out[1] = weight_grad(s[0], g[0]);
     return out;

@@ -267,6 +267,17 @@ class _StepProject(torch.autograd.Function):
         return dv, dg, None, (dz if ctx.masked else None), None, None
 
 
+@_host.gradient("noisy_point")
+def _noisy_point_grads(z, eps, dv):
+    return (torch.ops.ebr_fused.descent_noisy_point_bwd(z, dv, eps),)
+
+
+@_host.gradient("step_project")
+def _step_project_grads(v, g, alpha32, active8, rms, eps, dout):
+    dv, dg, dz = torch.ops.ebr_fused.descent_step_project_bwd(v, g, alpha32, active8, rms, dout, eps)
+    return dv, dg, None, None if active8 is None else dz
+
+
 # ---------------------------------------------------------------------------------------------------------------------
 # Reference-shaped entry points
 # ---------------------------------------------------------------------------------------------------------------------

@@ -336,6 +336,14 @@ def _skips_unused(q: Tensor) -> bool:
     return route(q.device) == "hip"
 
 
+def _second_grads(q, k, v, o, lse, do, dq, scale, gq, gk, gv):
+    """Gradients of (dq, dk, dv) for q, k, v, o, lse and do; o and lse are treated as constants: their dependence is
+    folded into hq / hk / hv / hdo."""
+    cot = [_zero_rows(ref) if g is None else g.to(ref.dtype) for g, ref in ((gq, q), (gk, k), (gv, v))]
+    hq, hk, hv, hdo = torch.ops.ebr_fused.attn_bwd_bwd(q, k, v, o, lse, do, dq, *cot, scale)
+    return hq, hk, hv, None, None, hdo
+
+
 class _FusedAttnBwd(torch.autograd.Function):
     """First derivative as a differentiable node: forward is attn_bwd, backward is attn_bwd_bwd."""
 
@@ -354,10 +362,7 @@ class _FusedAttnBwd(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gq, gk, gv):
         q, k, v, o, lse, do, dq = ctx.saved_tensors
-        cot = [_zero_rows(ref) if g is None else g.to(ref.dtype) for g, ref in ((gq, q), (gk, k), (gv, v))]
-        hq, hk, hv, hdo = torch.ops.ebr_fused.attn_bwd_bwd(q, k, v, o, lse, do, dq, *cot, ctx.scale)
-        # o and lse are treated as constants: their dependence is folded into hq / hk / hv / hdo.
-        return hq, hk, hv, None, None, hdo, None
+        return (*_second_grads(q, k, v, o, lse, do, dq, ctx.scale, gq, gk, gv), None)
 
 
 class _FusedAttn(torch.autograd.Function):
@@ -388,6 +393,16 @@ class _FusedAttn(torch.autograd.Function):
                 return None, None, None, None
             do = torch.zeros_like(o)
         return (*_FusedAttnBwd.apply(q, k, v, o, lse, do, ctx.scale), None)
+
+
+@_host.gradient("attention")
+def _attention_grads(q, k, v, o, lse, scale, do):
+    return _FusedAttnBwd.apply(q, k, v, o, lse, do, scale)
+
+
+@_host.gradient("attention_bwd")
+def _attention_bwd_grads(q, k, v, o, lse, do, scale, gq, gk, gv):
+    return _second_grads(q, k, v, o, lse, do, q, scale, gq, gk, gv)  # the op does not read its dq
 
 
 def _fused_attention_apply(q: Tensor, k: Tensor, v: Tensor, scale: float) -> Tensor:

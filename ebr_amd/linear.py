@@ -105,6 +105,19 @@ class _Linear(torch.autograd.Function):
         return dx, dw
 
 
+@_host.gradient("linear")
+def _linear_grads(x, w, dy, want_x, want_w):
+    return _Dgrad.apply(dy, w) if want_x else None, weight_grad(dy, x) if want_w else None
+
+
+@_host.gradient("linear_dgrad")
+def _dgrad_grads(dy, w, g, want_dy, want_w):
+    gdy = None
+    if want_dy:
+        gdy = _Linear.apply(g, w) if torch.is_grad_enabled() else F.linear(g, w)
+    return gdy, weight_grad(dy, g) if want_w else None
+
+
 def linear(x: Tensor, w: Tensor, b: Optional[Tensor] = None) -> Tensor:
     """F.linear(x, w, b) with split-K weight gradients (the bias, if any, added by torch)."""
     host = None if torch.compiler.is_compiling() else _host.module()

@@ -221,6 +221,132 @@ def test_modes_transforms_and_hooks_see_the_ops():
         torch.func.jvp(lambda x: fused_attention(x, k.detach(), v.detach()), (q.detach(),), (q.detach(),))
 
 
+def _rope_attn_case(dtype, device="cuda"):
+    """rope_attention of 2 heads of 32 on a 3 x 4 grid: (fn, inputs)."""
+    from ebr_amd.fused_attn.rope_split import rope_attention
+
+    cos, sin = (t.to(dtype) if dtype == torch.float64 else t for t in RotaryTable2D(32, 3, 4).to(device)())
+    xs = [_randn((2, 12, 192), dtype, 1, device), torch.tensor([0.7, 1.3], device=device)]
+    fn = rope_attention if device == "cuda" else _parts
+    return (lambda x, t: fn(x, cos, sin, 2, t)), xs
+
+
+def _grads_case(kind):
+    q = [_randn((2, 2, 9, 16), F32, i) for i in range(3)]
+    x = _randn((2, 12, 24), F32, 4)
+    if kind == "attn":
+        return fused_attention, q
+    if kind == "rope":
+        cos, sin = RotaryTable2D(4, 3, 4).cuda()()
+        return (lambda y: rope_split(y, cos, sin, 2)), [x]
+    if kind == "rope_attn":
+        return _rope_attn_case(F32)
+    if kind == "norm":
+        return (lambda y: block.rms_norm(y, 1e-5)), [x]
+    if kind == "add_norm":
+        return (lambda y, r: block.add_rms_norm(y, r, 1e-5)), [x, _randn(x.shape, F32, 5)]
+    if kind == "swiglu":
+        return block.swiglu, [x]
+    if kind == "linear":
+        return linear.linear, [x, _randn((5, 24), F32, 6)]
+    if kind == "noisy":
+        return (lambda z: descent.noisy_point(z, x, 0.3)), [x]
+    act = torch.tensor([True, False], device="cuda").view(2, 1, 1)
+    return (lambda v, g, z: descent.step_and_project(v, g, 0.1, z, act)), [_randn(x.shape, F32, i) for i in range(3)]
+
+
+KINDS = ["attn", "rope", "rope_attn", "norm", "add_norm", "swiglu", "linear", "noisy", "step"]
+
+
+def _nearly(a, b):
+    torch.testing.assert_close(a, b, rtol=2e-6, atol=2e-6 * b.abs().max().item())  # fp32 sums in another order
+
+
+@gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_batched_gradients(kind):
+    """A plain forward, then backwards under vmap: first derivatives, and the derivatives of recorded ones."""
+    fn, xs = _grads_case(kind)
+    xs = [x.detach().requires_grad_(True) for x in xs]
+    ys = fn(*xs)
+    ys = ys if isinstance(ys, tuple) else (ys,)
+    assert "CppNode" in ys[0].grad_fn.name()
+
+    def both(outs, wrt, seed):
+        cots = [_randn((3, *o.shape), o.dtype, seed + i) for i, o in enumerate(outs)]
+        got = torch.autograd.grad(outs, wrt, cots, is_grads_batched=True, retain_graph=True)
+        want = [torch.autograd.grad(outs, wrt, [c[i] for c in cots], retain_graph=True) for i in range(3)]
+        for i, g in enumerate(got):
+            _nearly(g, torch.stack([w[i] for w in want]))
+
+    both(ys, xs, 20)
+    if kind in ("noisy", "step"):  # first order only
+        return
+    cots = [_randn(y.shape, y.dtype, 30 + i).requires_grad_(True) for i, y in enumerate(ys)]
+    if kind == "rope_attn":  # its node of dx alone, and the one that records dt too
+        (dx,) = torch.autograd.grad(ys, xs[:1], cots, create_graph=True)
+        both([dx], [*xs, *cots], 40)
+        both([dx.square() + ys[0].repeat(1, 1, 3)], xs, 45)
+    first = torch.autograd.grad(ys, xs, cots, create_graph=True)
+    linear_in_x = kind in ("rope", "linear")  # no derivative of dx for x
+    both(first, cots if linear_in_x else [*xs, *cots], 50)
+
+
+@gpu
+def test_vectorised_jacobian_and_hessian():
+    q, k, v = (_randn((1, 1, 3, 16), F32, i) for i in range(3))
+    for strategy in (torch.autograd.functional.jacobian, torch.autograd.functional.hessian):
+        def fn(x):
+            y = block.swiglu(block.rms_norm(fused_attention(x, k, v), 1e-5))
+            return y if strategy is torch.autograd.functional.jacobian else y.square().sum()
+
+        _nearly(strategy(fn, q, vectorize=True), strategy(fn, q))
+
+
+@gpu
+def test_a_mode_around_the_backward_alone_sees_the_ops():
+    q, k, v = (_randn((1, 2, 9, 16), F32, i).requires_grad_(True) for i in range(3))
+    x = _randn((4, 16), F32, 3).requires_grad_(True)
+    o, n = fused_attention(q, k, v), block.swiglu(block.rms_norm(x, 1e-5))
+    with _Seen() as seen:
+        first = torch.autograd.grad([o, n], (q, k, v, x), [q.detach(), n.detach()], create_graph=True)
+        torch.autograd.grad(first, (q, k, v, x), [t.detach() for t in first])
+    for op in ("attn_bwd", "attn_bwd_bwd", "block_rmsnorm_bwd", "block_rmsnorm_bwd2", "block_swiglu_bwd",
+               "block_swiglu_bwd2"):
+        assert f"ebr_fused.{op}.default" in seen.ops
+    packed = []
+    o = fused_attention(q, k, v)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t, lambda t: t):
+        torch.autograd.grad(o, (q, k, v), q.detach(), create_graph=True)
+    assert len(packed) == 7
+
+
+def test_python_gradients_of_rope_attention():
+    """The formulas behind the native rope-attention node, on the CPU in 64 bits, against autograd of the parts."""
+    from ebr_amd.fused_attn import ops
+
+    fn, (x, t) = _rope_attn_case(torch.float64, "cpu")
+    cos, sin = (c.double() for c in RotaryTable2D(32, 3, 4)())
+    x, t = x.requires_grad_(True), t.double().requires_grad_(True)
+    dy = _randn((2, 12, 64), torch.float64, 3, "cpu").requires_grad_(True)
+    c = _randn((2, 12, 192), torch.float64, 4, "cpu")
+    want = torch.autograd.grad(fn(x, t), (x, t), dy, create_graph=True)
+    second = torch.autograd.grad(want[0], (x, t, dy), c)
+    q, k, v = rope_split(x, cos, sin, 2)
+    q = q * t.view(1, 2, 1, 1)
+    o, lse = torch.ops.ebr_fused.attn_fwd(q.detach(), k.detach(), v.detach(), 32**-0.5)
+    saved = [u.detach().requires_grad_(True) for u in (q, k, v)]
+    args = (t, *saved, dy, o, lse, cos, sin)
+    got = _host.GRADS["rope_attention"](x.detach(), t, cos, sin, *saved, o, lse, 32**-0.5, True, dy, None, None, None)
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=1e-9, atol=1e-9)
+    dq = ops._FusedAttnBwd.apply(*saved, o, lse, dy.reshape(2, 12, 2, 32).transpose(1, 2), 32**-0.5)[0]
+    dt, hq, hk, hv, hdy = _host.GRADS["rope_attention_bwd"](*args, dq, 32**-0.5, True, c)
+    dx, dt2 = _host.GRADS["rope_attention"](x.detach(), t, cos, sin, *saved, o, lse, 32**-0.5, True, None, hq, hk, hv)
+    for a, b in zip((dx, dt + dt2, hdy), second):
+        torch.testing.assert_close(a, b, rtol=1e-9, atol=1e-9)
+
+
 @gpu
 def test_refused_calls_stay_refused():
     q = _randn((1, 2, 9, 16), F32, 0)
