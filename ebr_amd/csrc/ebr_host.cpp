@@ -25,6 +25,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -694,9 +695,46 @@ struct RmsNormBwd : Function<RmsNormBwd> {
 // (the second derivative's) then come back to the forward node, whose own gradient kernel adds them.
 Tensor own_input(const Tensor& x) { return x.detach(); }
 
+// A second derivative alone passes through the forward node without using what it saved, and frees that where the caller
+// keeps no graph. With the input itself saved in the backward's node that pass would not come here at all, so it must
+// not use the node up: its saved input (output 1) is set aside for a later pass, until one uses it.
+struct Kept {
+    AutogradContext* ctx;
+    bool keeps = torch::autograd::get_current_graph_task_keep_graph();
+
+    Tensor use() {
+        const auto it = ctx->saved_data.find("kept");
+        if (it == ctx->saved_data.end()) {
+            const Tensor x = ctx->get_saved_variables()[0];  // an error where a pass has used it up
+            if (!keeps) ctx->saved_data["used"] = true;
+            return x;
+        }
+        const Tensor x = it->second.toTensor().detach();
+        TORCH_CHECK((int64_t)x._version() == ctx->saved_data["version"].toInt(),
+                    "one of the variables needed for gradient computation has been modified by an inplace operation");
+        if (const auto node = torch::autograd::get_current_node())
+            torch::autograd::impl::set_gradient_edge(x, {node, 1});
+        if (!keeps) ctx->saved_data.erase(it);
+        return x;
+    }
+    void pass() {
+        if (keeps || ctx->saved_data.count("kept") || ctx->saved_data.count("used")) return;
+        const Tensor x = ctx->get_saved_variables()[0].detach();
+        ctx->saved_data["version"] = (int64_t)x._version();
+        ctx->saved_data["kept"] = x;
+        ctx->saved_data["used"] = true;  // what the context itself saved goes with this pass
+    }
+};
+
 // The gradient of a norm's input: from dy through the backward's node, plus ``acc``.
-Tensor norm_grad(const Tensor& x, const Tensor& dy, const Tensor& acc, double eps) {
-    if (!dy.defined()) return acc;
+Tensor norm_grad(AutogradContext* ctx, const Tensor& dy, const Tensor& acc) {
+    Kept saved{ctx};
+    if (!dy.defined()) {
+        saved.pass();
+        return acc;
+    }
+    const Tensor x = saved.use();
+    const double eps = ctx->saved_data["eps"].toDouble();
     if (!native({dy, acc})) return python_grads("rms_norm", 1, x, eps, dy, acc)[0];
     if (acc.defined() && !at::GradMode::is_enabled()) return rmsnorm_bwd(x, dy, acc, eps);
     const Tensor dx = RmsNormBwd::apply(x, dy, eps)[0];
@@ -712,8 +750,7 @@ struct RmsNorm : Function<RmsNorm> {
         return {rmsnorm(x, eps), own};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-        const Tensor x = ctx->get_saved_variables()[0];
-        return {norm_grad(x, g[0], g[1], ctx->saved_data["eps"].toDouble()), Tensor()};
+        return {norm_grad(ctx, g[0], g[1]), Tensor()};
     }
 };
 
@@ -726,8 +763,7 @@ struct AddRmsNorm : Function<AddRmsNorm> {
         return {out[1], out[0]};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-        const Tensor x = ctx->get_saved_variables()[0];
-        const Tensor d = norm_grad(x, g[0], g[1], ctx->saved_data["eps"].toDouble());
+        const Tensor d = norm_grad(ctx, g[0], g[1]);
         return {d, d, Tensor()};
     }
 };
@@ -801,8 +837,12 @@ struct SwiGLU : Function<SwiGLU> {
         return {swiglu_fwd(gu), own};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-        if (!g[0].defined()) return {g[1]};
-        const Tensor gu = ctx->get_saved_variables()[0];
+        Kept saved{ctx};
+        if (!g[0].defined()) {
+            saved.pass();
+            return {g[1]};
+        }
+        const Tensor gu = saved.use();
         if (!native(g)) return python_grads("swiglu", 1, gu, g[0], g[1]);
         if (g[1].defined() && !at::GradMode::is_enabled()) return {swiglu_bwd(gu, g[0], g[1])};
         const Tensor d = SwiGLUBwd::apply(gu, g[0])[0];

@@ -180,6 +180,56 @@ def test_plain_calls_take_it():
 
 
 @gpu
+@pytest.mark.parametrize("path,kind", [("native", "norm"), ("native", "add_norm"), ("native", "swiglu"),
+                                       ("python", "norm"), ("python", "swiglu")])
+def test_a_second_derivative_alone_leaves_the_forward_node_usable(monkeypatch, kind, path):
+    if path == "python":
+        monkeypatch.setattr(_host, "module", lambda: None)
+    x0, r = _randn((3, 5, 24), F32, 1), _randn((3, 5, 24), F32, 2)
+    fn = {"norm": lambda x: block.rms_norm(x, 1e-5), "swiglu": block.swiglu,
+          "add_norm": lambda x: block.add_rms_norm(x, r, 1e-5)}[kind]
+
+    def graph():
+        x = x0.clone().requires_grad_(True)
+        z = x * 1
+        y = fn(z)
+        dy = _randn(y.shape, F32, 3)
+        (g,) = torch.autograd.grad(y, z, dy, create_graph=True)
+        return z, y, dy, g
+
+    def first(y, z, dy, **kw):
+        return torch.autograd.grad(y, z, dy, **kw)[0]
+
+    z, y, dy, g = graph()
+    h = first(g, z, x0)
+    assert torch.equal(first(y, z, dy, create_graph=True), g)  # still there, once more and recorded
+    again = first(y, z, dy, create_graph=True)
+    assert torch.equal(first(again, z, x0), h)
+    assert torch.equal(first(y, z, dy), g)  # and this pass uses it up
+    with pytest.raises(RuntimeError, match="second time"):
+        first(y, z, dy)
+    z, y, dy, g = graph()
+    assert torch.equal(first(y, z, dy), g)  # used up by the first derivative: the recorded gradient has its own
+    assert torch.equal(first(g, z, x0), h)
+    with pytest.raises(RuntimeError, match="second time"):
+        first(y, z, dy)
+    del z, y, dy, g, h, again
+    before = torch.cuda.memory_allocated()
+    z, y, dy, g = graph()
+    first(g, z, x0)
+    assert torch.cuda.memory_allocated() > before
+    del z, y, dy, g  # what was set aside goes with the graph
+    assert torch.cuda.memory_allocated() == before
+    if kind != "add_norm":  # the sum is no tensor of the caller's
+        z, y, dy, g = graph()
+        first(g, z, x0)
+        with torch.no_grad():
+            z.add_(1)
+        with pytest.raises(RuntimeError, match="inplace"):
+            first(y, z, dy)
+
+
+@gpu
 def test_no_derivative_past_the_second():
     x = _randn((4, 16), F32, 0).requires_grad_(True)
     (g,) = torch.autograd.grad(block.rms_norm(x, 1e-5).square().sum(), x, create_graph=True)
