@@ -361,6 +361,52 @@ def test_verify_second_order_rejects_backend_without_second_derivative():
         att.verify_second_order(bad, device=torch.device("cpu"))
 
 
+def _rope_parts(qkv, cos, sin, heads, t):
+    from ebr_amd.fused_attn.rope_split import dense_split
+
+    q, k, v = dense_split(qkv, cos, sin, cos.new_zeros((0,)), heads)
+    return att.math_attention(q * t.view(1, heads, 1, 1), k, v).transpose(1, 2).reshape(*qkv.shape[:2], -1)
+
+
+def _rope_detached_temperature(qkv, cos, sin, heads, t):  # right values, no gradient of the gradient for t
+    return _rope_parts(qkv, cos, sin, heads, t.detach()) + 0 * t.sum()
+
+
+def _rope_planted(qkv, cos, sin, heads, t):  # right first derivatives for z, second ones of another function
+    y = _rope_parts(qkv, cos, sin, heads, t)
+    w = qkv - qkv.detach()
+    return y + w[..., : y.shape[-1]].pow(2)
+
+
+def test_graded_blocks_test_the_node_that_serves_them(monkeypatch):
+    """Behind the fused RoPE split one node takes the backend's place: a graded call tests it before it uses it."""
+    from ebr_amd.fused_attn import rope_split
+    from ebr_amd.layers import RotaryTable2D
+
+    rope = RotaryTable2D(16, 3, 3)()
+
+    def call(fn, graded=True):
+        monkeypatch.setattr(rope_split, "rope_attention", fn)
+        torch.manual_seed(0)
+        layer = att.EnergyAttention(32, 16, 2, backend="fused", nograd_backend="fused")
+        layer._verified = True  # the backend's own test has its own cases
+        x = torch.randn(2, 9, 32)
+        drawn = torch.get_rng_state()
+        with att.second_order_window(graded):
+            y = layer(rope, x)
+        assert torch.equal(torch.get_rng_state(), drawn)
+        return layer, y
+
+    layer, y = call(_rope_parts)
+    assert layer._node_verified
+    layer, parts = call(lambda *a: None)  # the parts serve the call: nothing to test
+    assert not layer._node_verified and torch.allclose(parts, y, atol=1e-6)
+    for wrong in (_rope_detached_temperature, _rope_planted):
+        with pytest.raises(att.SecondOrderUnsafeError, match="rope_attention"):
+            call(wrong)
+    assert not call(_rope_planted, graded=False)[0]._node_verified
+
+
 def test_self_test_priming_keeps_the_global_rng_and_seeding_reaches_every_layer():
     """prime_attention_self_test runs each layer's self-test once under a forked RNG (the caller's next draw is
     unchanged); seed_attention_self_test sets the seed the pending self-tests will use."""

@@ -520,6 +520,23 @@ def test_rope_attention_is_its_parts(dtype, B, grid, H, D):
 
 
 @gpu
+@pytest.mark.parametrize("dtype,head_dim", [(BF16, 32), (F32, 16)])
+def test_graded_blocks_test_rope_attention_first(dtype, head_dim):
+    from ebr_amd import attention
+
+    layer = attention.EnergyAttention(2 * head_dim, head_dim, 2, backend="fused", nograd_backend="fused").cuda()
+    rope = RotaryTable2D(head_dim, 3, 3).cuda()()
+    x = _randn((2, 9, 2 * head_dim), dtype, 1)
+    layer(rope, x)
+    assert not layer._node_verified
+    with attention.second_order_window(True):
+        layer(rope, x)
+    assert layer._verified and layer._node_verified
+    with _Seen():  # the parts run: nothing to test
+        assert not attention.verify_rope_attention(device=x.device)
+
+
+@gpu
 def test_rope_attention_leaves_other_calls():
     from ebr_amd.fused_attn.rope_split import rope_attention
 
