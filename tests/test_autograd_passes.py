@@ -1,5 +1,6 @@
 """How often the attention ops run in a derivative: on the GPU a node that gets no cotangent launches nothing. The CPU
-cases take the GPU's rule over the dense path."""
+cases take the GPU's rule over the dense path; the GPU cases run under the rule itself, on the Python nodes (a mode counts
+their ops) and on the native ones (a profiler counts their ranges)."""
 
 import pytest
 import torch
@@ -31,13 +32,30 @@ def _inputs(n=7, device="cpu"):
 
 
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
-def test_second_derivative_runs_each_op_once(gpu_rule, device):
+def test_second_derivative_runs_each_op_once(request, device):
+    if device == "cpu":
+        request.getfixturevalue("gpu_rule")
     (q, k, v, do), cot = _inputs(device=device)
     with _Count() as seen:
         o = fused_attention(q, k, v)
         first = torch.autograd.grad(o, (q, k, v), do, create_graph=True)
         torch.autograd.grad(first, (q, k, v, do), cot)
     assert seen.calls == ["attn_fwd", "attn_bwd", "attn_bwd_bwd"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_native_second_derivative_runs_each_op_once(dtype):
+    g = torch.Generator().manual_seed(3)
+    q, k, v, do, *cot = (torch.randn((2, 2, 9, 16), generator=g).to("cuda", dtype).requires_grad_(i < 4)
+                         for i in range(7))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        o = fused_attention(q, k, v)
+        first = torch.autograd.grad(o, (q, k, v), do, create_graph=True)
+        torch.autograd.grad(first, (q, k, v, do), cot)
+    assert "CppNode" in o.grad_fn.name()
+    counts = {e.key: e.count for e in prof.key_averages() if e.key.startswith("ebr_fused::")}
+    assert counts == {"ebr_fused::attn_fwd": 1, "ebr_fused::attn_bwd": 1, "ebr_fused::attn_bwd_bwd": 1}
 
 
 def test_second_derivative_with_a_use_of_the_output_runs_the_backward_again(gpu_rule):
