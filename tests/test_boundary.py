@@ -399,6 +399,10 @@ def test_graded_blocks_test_the_node_that_serves_them(monkeypatch):
 
     layer, y = call(_rope_parts)
     assert layer._node_verified
+    vars(layer).pop("_node_verified")  # as a module pickled before the attribute was there
+    with att.second_order_window(True):
+        layer(rope, torch.randn(2, 9, 32))
+    assert layer._node_verified
     layer, parts = call(lambda *a: None)  # the parts serve the call: nothing to test
     assert not layer._node_verified and torch.allclose(parts, y, atol=1e-6)
     for wrong in (_rope_detached_temperature, _rope_planted):
