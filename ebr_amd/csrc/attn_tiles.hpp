@@ -60,10 +60,10 @@ struct f32n {
 // that of a bf16 2^-133 (the bf16 MFMA and the conversion keep subnormals; without the scale the small parts of an
 // |x| < 2^-110 lost bits, 2^-9 of x itself near 2^-126). |mid| <= 2^-8 |hi|, |lo| <= 2^-16 |hi|. A product of two
 // values is the six products of parts down to 2^-16 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the three left
-// out are below 2^-23 of it at worst and 2^-27 in the mean, of either sign. Each product of parts is exact in the MFMA's fp32,
-// and the small ones enter an accumulator first. Sums carry 2^32, which leaves at the end of a sum. Six bf16 MFMAs of
-// k = 32 take 96 cycles where eight fp32 MFMAs of k = 4 take 256, and a plane is read transposed, so a tensor is staged
-// once instead of natural and transposed. Measured at B H = 64, L = 400, D = 64 (fp32 MFMA -> split): forward
+// out are below 2^-23 of it at worst and 2^-27 in the mean, of either sign. Each product of parts is exact in the MFMA's
+// fp32, and the small ones enter an accumulator first. Sums carry 2^32, which leaves at the end of a sum. Six bf16 MFMAs
+// of k = 32 take 96 cycles where eight fp32 MFMAs of k = 4 take 256, and a plane is read transposed, so a tensor is
+// staged once instead of natural and transposed. Measured at B H = 64, L = 400, D = 64 (fp32 MFMA -> split): forward
 // 45 -> 36, backward 126 -> 90, bwd_bwd 329 -> 190 us, the error against 64 bits 4.6e-7 -> 3.3e-7, 5.9e-7 -> 4.8e-7,
 // 7.2e-7 -> 5.9e-7 (fewer roundings per sum). A sum that is one product alone is less exact than on the fp32 MFMA: at
 // worst 9.9e-8 of it instead of 6.0e-8, 2.6e-8 instead of 2.5e-8 in the root mean square. The two products of 2^-24
@@ -71,7 +71,8 @@ struct f32n {
 // accumulator for each scale, cost 16% (39, 107, 221 us).
 // A non-finite input, or one past 2^111, does not survive the split: it gives NaN wherever it enters, and a sum past
 // 2^96 overflows. A workgroup with a sum that is not finite computes it again with f32n (see redo_unsplit), so the
-// results for such inputs are those of plain fp32 arithmetic.
+// results for such inputs are those of plain fp32 arithmetic. Where only the backward does so, its P differs from the
+// forward's by the scores' roundings: up to three times the error of either side (2e-6 to 3e-6 at scores of about 100).
 constexpr int NPLANE = 3;
 constexpr float PLANE_SCALE = 0x1p16f, PRODUCT_UNSCALE = 0x1p-32f;  // of a value's planes; off a product of two
 
